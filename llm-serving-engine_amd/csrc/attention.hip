@@ -10,6 +10,9 @@
 // Like the reference, the softmax runs online in fp32 and the probabilities are rounded to bf16
 // before the product with V (fp32 accumulation); the output is rounded to bf16.
 //
+// This kernel streams the keys past few query rows: decode rows and short chunks. Longer entries are
+// attn_tile.hip's (attn_is_long, attention.h).
+//
 // Work decomposition. A workgroup of four waves takes one (entry, K/V head, query tile) item, or
 // one key chunk of it. A query tile is 16 MFMA rows: TQ = floor(16 / G) query tokens x the G query
 // heads that share the K/V head (GQA), so every K/V byte a workgroup reads serves all G heads; with
@@ -39,7 +42,7 @@
 //    four keys kb..kb+3 at column d0 + i: exactly the B operand for those keys.
 #include <algorithm>
 
-#include "lse_common.h"
+#include "attention.h"
 
 namespace lse {
 
@@ -52,41 +55,6 @@ constexpr int kAttnKeys = 32;     // keys per wave tile
 constexpr int kAttnChunk = 1024;
 constexpr int kAttnMaxSplit = 64;  // chunks per item the split launch takes at most
 static_assert(kAttnChunk % (kAttnWaves * kAttnKeys) == 0, "whole rounds of wave tiles per chunk");
-
-struct PagedAttnArgs {
-  const uint16_t* q;  // bf16, element (h, t, d) at h * sq_h + t * sq_t + d
-  int64_t sq_h, sq_t;
-  const uint16_t* k_pool;  // bf16 (blocks, block_size, H_KV, D): (b, w, h, d) at b sb + w sw + h sh + d
-  const uint16_t* v_pool;
-  int64_t sb, sw, sh;
-  const int32_t* block_table;  // (entries, max_blocks), row stride sbt
-  int64_t sbt;
-  const int32_t* context_len;
-  const int32_t* query_offset;
-  const int32_t* q_start;
-  const int32_t* q_len;
-  uint16_t* o;  // bf16, same indexing as q with strides so_h, so_t
-  int64_t so_h, so_t;
-  int entries, H, HKV, G, block_size, max_q_len;
-  int bs_shift;      // log2(block_size) when it is a power of two, else -1
-  int tq;            // query tokens per tile: floor(16 / G)
-  int qtiles;        // ceil(max_q_len / tq)
-  int parts;         // 1: a workgroup folds every chunk of its item; > 1: one chunk per workgroup
-  float scale_log2;  // softmax scale x log2(e): scores are kept in the base-2 domain
-  float* ws_o;       // parts > 1: chunk states' O [parts][entries][H][max_q_len][D], fp32
-  float* ws_ml;      // parts > 1: chunk states' max and sum [parts][entries][H][max_q_len][2]
-};
-
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
-// 16-lane transposing LDS read (see the header comment).
-__device__ __forceinline__ bf16x4 lds_read_tr16(const unsigned char* p) {
-  typedef __attribute__((address_space(3))) bf16x4* LdsV4;
-  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-      (LdsV4)((__attribute__((address_space(3))) unsigned char*)p));
-}
-
-__device__ __forceinline__ float exp2_fast(float v) { return __builtin_amdgcn_exp2f(v); }
 
 // The tile's causal bound: the furthest position any of its rows attends to is query_offset +
 // min(q_len, (qt + 1) * TQ) - 1, and never past context_len. Keys [0, attn_end) are its chunks'.
@@ -146,17 +114,22 @@ paged_attn_kernel(PagedAttnArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, grp = lane >> 4;
 
+  // K/V heads run fastest and query tiles slowest: consecutive workgroups go to the 8 XCDs in turn,
+  // and of a mixed batch only the first tile of most entries (and, split, the first chunks) exists.
+  // With tiles or chunks fastest, 16 tiles put all decode rows on one XCD.
   int b = blockIdx.x;
-  const int part = b % a.parts;
-  b /= a.parts;
-  const int qt = b % a.qtiles;
-  b /= a.qtiles;
   const int kvh = b % a.HKV;
-  const int e = b / a.HKV;
+  b /= a.HKV;
+  const int e = b % a.entries;
+  b /= a.entries;
+  const int part = b % a.parts;
+  const int qt = b / a.parts;
   const int G = a.G, TQ = a.tq;
   const int qlen = a.q_len[e];
   if (qt * TQ >= qlen) return;
-  const int ctx = a.context_len[e], qo = a.query_offset[e], qs = a.q_start[e];
+  const int ctx = a.context_len[e];
+  if (a.tiled && attn_is_long((int64_t)qlen * G, ctx)) return;
+  const int qo = a.query_offset[e], qs = a.q_start[e];
   const int end_n = attn_end(qo, qlen, ctx, qt, TQ);
   const int nch = attn_chunks(end_n);
   // Split launch: this workgroup's chunk only (none past the tile's keys: the fold reads no
@@ -385,6 +358,7 @@ paged_attn_merge(PagedAttnArgs a) {
   const int e = (int)(r / a.H);
   const int qlen = a.q_len[e];
   if (m >= qlen) return;
+  if (a.tiled && attn_is_long((int64_t)qlen * a.G, a.context_len[e])) return;
   const int end_n = attn_end(a.query_offset[e], qlen, a.context_len[e], m / a.tq, a.tq);
   const int np = attn_chunks(end_n);
   const int64_t stride = (int64_t)a.entries * a.H * a.max_q_len;
@@ -402,6 +376,8 @@ paged_attn_merge(PagedAttnArgs a) {
 
 struct AttnPlan {
   int tq, qtiles, parts;
+  bool tiled;       // some entry may be the row-tiled kernel's
+  int64_t short_q;  // the most query rows of an entry that is not
   int64_t ws_o_bytes, ws_bytes;
 };
 
@@ -412,15 +388,18 @@ struct AttnPlan {
 static AttnPlan attn_plan(int64_t entries, int64_t H, int64_t HKV, int64_t D, int64_t max_q_len,
                           int64_t max_ctx, int cus) {
   AttnPlan pl{};
+  const int64_t G = H / HKV;
+  pl.tiled = max_q_len * G >= kAttnTileRows;
+  pl.short_q = std::min<int64_t>(max_q_len, (kAttnTileRowsFar - 1) / G);
   pl.tq = (int)(16 / (H / HKV));
-  pl.qtiles = (int)ceil_div(max_q_len, pl.tq);
+  pl.qtiles = (int)ceil_div(pl.short_q, pl.tq);
   const int64_t items = entries * HKV * pl.qtiles;
   const int64_t chunks = ceil_div(std::max<int64_t>(max_ctx, 1), kAttnChunk);
   pl.parts = items > 0 && items < 2 * (int64_t)cus && chunks > 1 && chunks <= kAttnMaxSplit
                  ? (int)chunks
                  : 1;
   if (pl.parts > 1) {
-    const int64_t slots = (int64_t)pl.parts * entries * H * max_q_len;
+    const int64_t slots = (int64_t)pl.parts * entries * H * pl.short_q;
     pl.ws_o_bytes = slots * D * 4;
     pl.ws_bytes = pl.ws_o_bytes + slots * 2 * 4;
   }
@@ -487,7 +466,14 @@ int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const 
   a.ws_o = pl.parts > 1 ? static_cast<float*>(ws) : nullptr;
   a.ws_ml = pl.parts > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + pl.ws_o_bytes) : nullptr;
   const int64_t blocks = (int64_t)a.entries * a.HKV * pl.qtiles * pl.parts;
-  if (blocks > 0x7fffffff) return LSE_E_RANGE;
+  if (blocks > 0x7fffffff ||
+      (int64_t)a.entries * a.HKV * ceil_div(max_q_len, pl.tq) > 0x7fffffff)
+    return LSE_E_RANGE;
+  a.tiled = pl.tiled;
+  if (pl.tiled) {
+    if (int st = launch_attn_tile(a, attn_cus(), stream)) return st;
+    a.max_q_len = (int)pl.short_q;
+  }
   void* args[] = {&a};
   const bool pow2 = a.bs_shift >= 0;
   const void* fn =

@@ -1,0 +1,85 @@
+"""The row-tiled paged attention of long entries on the GPU against the fp64 oracle, where it can go
+wrong: the first entry length it takes, tiles of 128 rows and 64 keys one short and one over, groups
+that do not divide a tile, block sizes a wave's 16 keys do and do not fit, short entries beside
+long ones. The tolerance is test_gpu_attention's (bf16 probabilities and output)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gpu_attention import _case, _check, _run
+
+pytestmark = pytest.mark.gpu
+
+FIRST_ROWS = 256  # query rows (tokens x heads of a K/V head) from which an entry is row-tiled...
+NEAR = 2048  # ...when its context is no longer than this; from twice the rows on in any case
+
+
+@pytest.mark.parametrize("h,h_kv", [(4, 4), (6, 2), (8, 2), (10, 2), (16, 1)])
+def test_first_length_and_tile_edges(pkg, dev, h, h_kv):
+    """Entries on both sides of the first row-tiled length, and of the next row tile."""
+    g = h // h_kv
+    first = -(-FIRST_ROWS // g)
+    lens = [first - 1, first, first + 1, (FIRST_ROWS + 128) // g, (FIRST_ROWS + 128) // g + 1]
+    entries = [(n, off, n + off) for n, off in zip(lens, [0, 0, 3, 64, 129])]
+    _check(pkg, dev, _case(100 + h, entries, h=h, h_kv=h_kv), f"H={h} H_KV={h_kv}")
+
+
+def test_far_chunks_start_later(pkg, dev):
+    """Entries on both sides of the context and row bounds, whose tiles span many key steps."""
+    entries = [(n, ctx - n, ctx) for n in (32, 63, 64) for ctx in (NEAR, NEAR + 1)]
+    _check(pkg, dev, _case(150, entries, h=8, h_kv=1), "far chunks")
+
+
+@pytest.mark.parametrize("end", [63, 64, 65, 127, 128, 129, 191, 192, 193, 257])
+def test_key_tile_edges(pkg, dev, end):
+    """Contexts one short of and one over a key tile, a pair of tiles and the four in flight; the
+    second entry's context ends before its own query rows do, so its rows see different ends."""
+    c = _case(200 + end, [(end, 0, end), (end, 11, end)], h=16, h_kv=2)
+    _check(pkg, dev, c, f"end={end}")
+
+
+@pytest.mark.parametrize("block_size", [1, 7, 16, 24, 48, 64])
+def test_block_sizes(pkg, dev, block_size):
+    entries = [(150, 77, 227), (1, 300, 301), (64, 0, 64), (5, 100, 105)]
+    _check(pkg, dev, _case(300 + block_size, entries, h=8, h_kv=2, block_size=block_size),
+           f"block {block_size}")
+
+
+def test_rows_that_see_no_key(pkg, dev):
+    """An entry without any context gives zeros."""
+    c = _case(400, [(70, 0, 70), (80, 0, 80)], h=8, h_kv=2)
+    c["ctx"] = np.array([70, 0], np.int32)
+    o = _run(pkg, dev, c)
+    assert not (o[:, 70:] & 0x7FFF).any()
+    assert (o[:, :70] & 0x7FFF).any()
+
+
+def test_rows_do_not_depend_on_the_batch(pkg, dev):
+    """A long entry's rows have the same bits alone, among decode rows and other prompts, with a
+    larger max_q_len and a wider table; slots nobody owns hold NaN."""
+    entries = [(1, 40, 41), (200, 100, 300), (90, 0, 90), (1, 700, 701), (65, 31, 96)]
+    c = _case(500, entries, h=8, h_kv=2, spare_blocks=5)
+    base = _check(pkg, dev, c, "batch")
+    owned = np.zeros(c["kp"].shape[:2], bool)
+    for e, ctx in enumerate(c["ctx"]):
+        for n in range(ctx):
+            owned[c["table"][e][n // c["bs"]], n % c["bs"]] = True
+    kp, vp = c["kp"].copy(), c["vp"].copy()
+    kp[~owned] = vp[~owned] = np.uint16(0x7FC0)
+    np.testing.assert_array_equal(_run(pkg, dev, c, kp, vp), base, err_msg="NaN elsewhere")
+    for e in (1, 2, 4):
+        rows = slice(c["qs"][e], c["qs"][e] + c["ql"][e])
+        pick = lambda a: a[e:e + 1]  # noqa: E731
+        one = dict(c, q=c["q"][:, rows].copy(), table=np.pad(pick(c["table"]), ((0, 0), (0, 900))),
+                   ctx=pick(c["ctx"]), qo=pick(c["qo"]), ql=pick(c["ql"]),
+                   qs=np.zeros(1, np.int32), max_q_len=4000)
+        np.testing.assert_array_equal(_run(pkg, dev, one), base[:, rows], err_msg=f"entry {e}")
+
+
+def test_more_entries_than_one_launch_holds(pkg, dev):
+    """Over 1024 entries, a few of them long."""
+    entries = [(17 if e % 100 == 0 or e > 1026 else 1, 0, 17 if e % 100 == 0 or e > 1026 else 1)
+               for e in range(1030)]
+    _check(pkg, dev, _case(600, entries, h=16, h_kv=1), "1030 entries")

@@ -84,10 +84,11 @@ enum lse_query_key {
   LSE_Q_NOALLOC_SCRATCH = 5, /* bytes of the static scratch lse_w8a16_gemm_noalloc works in */
 };
 
-#define LSE_ABI_VERSION 12
+#define LSE_ABI_VERSION 13
 #define LSE_NOALLOC_SCRATCH_BYTES (32 << 20)
 #define LSE_K_ALIGN 16
 #define LSE_DECODE_MAX_M 64
+#define LSE_NORM_MAX_K 16384  /* longest row of lse_add_rmsnorm */
 #define LSE_MAX_K 133120      /* 127*127*K < 2^31 with margin; multiple of LSE_K_ALIGN */
 
 /*
@@ -330,6 +331,43 @@ int lse_pack_bf16_weight(const void* w, int64_t ldw, int64_t N, int64_t K, void*
  */
 int lse_bf16_decode_gemm(const void* x, int64_t ldx, const void* wp, void* y, int64_t ldy,
                          int64_t M, int64_t N, int64_t K, void* stream);
+
+/*
+ * The residual addition and the RMSNorm after it, one pass over each row:
+ *   s[m,k] = bf16(x[m,k] + res[m,k])  (x itself when res is NULL),
+ *   r = 1 / sqrt(fl32(sum_k s[m,k]^2 / K) + eps),  y[m,k] = bf16(weight[k] * bf16(s[m,k] * r)),
+ * the roundings of LlamaRMSNorm; the sum of squares runs in a fixed fp32 order.
+ * x, res: (M, K) bf16, row strides ldx, ldr (multiples of 8, 16-byte aligned). weight: (K) bf16.
+ * sum: (M, K) bf16 contiguous receiving s, or NULL; it may be x or res when that is contiguous.
+ * y: (M, K) bf16 contiguous, no other argument's memory. K % 8 == 0, K <= LSE_NORM_MAX_K.
+ * Replaces: `hidden + ...` and the norm that reads it in `decoder_hidden`
+ * (model_runner.py:222-223; LlamaRMSNorm.forward, modeling_llama.py:62-67).
+ */
+int lse_add_rmsnorm(const void* x, int64_t ldx, const void* res, int64_t ldr, const void* weight,
+                    float eps, void* sum, void* y, int64_t M, int64_t K, void* stream);
+
+/*
+ * Rotary embedding of one layer's new q and k rows, and their K/V writes, in one launch. Token t =
+ * sequence t / tokens_per_sequence, position start + t % tokens_per_sequence. With c, s the row t of
+ * cos and sin and x a head's row, out[d] = bf16(bf16(x[d] c[d]) + bf16(rot[d] s[d])), rot[d] =
+ * -x[d + D/2] for d < D/2 and x[d - D/2] above, bit for bit what apply_rotary_pos_emb gives in bf16.
+ * q, k, v: bf16 rows of H x D, H_KV x D and H_KV x D values, row strides q_stride, k_stride,
+ *   v_stride. cos, sin: (tokens, D) bf16, row stride cs_stride. q_out: (tokens, H, D) bf16.
+ * k_cache, v_cache: contiguous-per-head caches, element (sequence, head, position, d); pools:
+ *   element (block, slot, head, d), position p of sequence e in block block_table[e][p /
+ *   block_size], slot p % block_size. Either pair may be NULL. The table's values must lie in the
+ *   pool and name distinct slots for distinct tokens.
+ * D % 16 == 0, strides multiples of 8, 16-byte aligned pointers, at most 65535 tokens.
+ * Replaces: apply_rotary_pos_emb and the K/V writes in `_project_qkv` and `attend_paged`
+ * (model_runner.py:310-363).
+ */
+int lse_rope_kv(const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                int64_t v_stride, const void* cos, const void* sin, int64_t cs_stride, void* q_out,
+                void* k_cache, void* v_cache, int64_t cache_stride_seq, int64_t cache_stride_head,
+                int64_t cache_stride_pos, void* k_pool, void* v_pool, int64_t pool_stride_block,
+                int64_t pool_stride_slot, int64_t pool_stride_head, const int32_t* block_table,
+                int64_t block_table_stride, int64_t block_size, int64_t H, int64_t H_KV, int64_t D,
+                int64_t sequences, int64_t tokens_per_sequence, int64_t start, void* stream);
 
 /* Static properties (enum lse_query_key); -1 for an unknown key. Load-time checks read these,
  * as `ModelRunner.check_custom_kernel_support` (model_runner.py:77-94) checks its kernels. */

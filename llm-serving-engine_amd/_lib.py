@@ -42,6 +42,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "lse_paged_attention": (_INT, [_P, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P,
                                    _P, _P, _I64, _I64] + [_I64] * 7 + [ctypes.c_float, _P, _I64,
                                                                         _P]),
+    "lse_add_rmsnorm": (_INT, [_P, _I64, _P, _I64, _P, ctypes.c_float, _P, _P, _I64, _I64, _P]),
+    "lse_rope_kv": (_INT, [_P, _I64] * 3 + [_P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _P, _P]
+                    + [_I64] * 3 + [_P] + [_I64] * 8 + [_P]),
     "lse_query": (_I64, [_INT]),
     "lse_status_string": (ctypes.c_char_p, [_INT]),
 }
@@ -53,7 +56,8 @@ MODE_W8A16, MODE_W8A8 = 0, 1
 E_WORKSPACE, E_SCRATCH = -6, -7
 Q_ABI_VERSION, Q_K_ALIGN, Q_DECODE_MAX_M, Q_MAX_K, Q_GFX_ARCH = 0, 1, 2, 3, 4
 Q_NOALLOC_SCRATCH = 5
-ABI_VERSION = 12
+ABI_VERSION = 13
+NORM_MAX_K = 16384
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

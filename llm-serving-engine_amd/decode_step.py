@@ -23,6 +23,8 @@ applies o_proj (`attention_output`, model_runner.py:365-369).
     per-token quantization, exact integer sums and (acc·sx)·s; gate/up as fp32 g and u with
     silu(g)·u rounded once, as the fused kernel rounds it); it isolates the kernels from the
     quantization itself. Test and measurement use only.
+On the GPU the rotary embedding with its K/V writes (`ops.rope_kv`) and each residual addition with
+the norm after it (`ops.add_rmsnorm`) run as one kernel each, in every back end.
 With `trace` set to a list, every int8 projection of a step appends (layer, name, input,
 output), so each layer's kernels can be checked on the very input they saw (errors do not
 compound over layers).
@@ -44,7 +46,7 @@ import math
 import torch
 from torch import nn
 
-from . import ops
+from . import _lib, ops
 from .int8_linear import Int8GateUp, Int8Linear, PackedBf16Linear
 
 LLAMA3_8B = dict(
@@ -133,17 +135,21 @@ class DecodeRunner:
         self.k_pool[i][blocks, within] = k.transpose(1, 2)
         self.v_pool[i][blocks, within] = v.transpose(1, 2)
 
-    def _attend_paged(self, i: int, q: torch.Tensor, start: int, end: int, nseq: int,
-                      ntok: int) -> torch.Tensor:
-        """q (nseq, H, ntok, D) -> (1, nseq * ntok, H * D) through one paged attention launch."""
-        dev = q.device
-        qh = q.permute(1, 0, 2, 3).reshape(self.n_heads, nseq * ntok, self.head_dim).contiguous()
-        table = self.tables[self._rows].contiguous()
+    def _attend_paged(self, i: int, q: torch.Tensor) -> torch.Tensor:
+        """q (nseq * ntok, H, D) -> (1, nseq * ntok, H * D) through one paged attention launch; the
+        output comes in q's own token-major layout."""
+        table, ctx, offset, q_start, q_len, ntok = self._plan
+        o = ops.paged_attention_forward(q.transpose(0, 1), self.k_pool[i], self.v_pool[i], table, ctx,
+                                        offset, q_start, q_len, self.block_size, ntok)
+        return o.transpose(0, 1).reshape(1, q.shape[0], self.n_heads * self.head_dim)
+
+    def _paged_plan(self, start: int, end: int, nseq: int, ntok: int):
+        """The paging tensors every layer of one call shares."""
+        dev = self.k_cache[0].device
         full = lambda v: torch.full((nseq,), v, dtype=torch.int32, device=dev)  # noqa: E731
         q_start = torch.arange(0, nseq * ntok, ntok, dtype=torch.int32, device=dev)
-        o = ops.paged_attention_forward(qh, self.k_pool[i], self.v_pool[i], table, full(end),
-                                        full(start), q_start, full(ntok), self.block_size, ntok)
-        return o.permute(1, 0, 2).reshape(1, nseq * ntok, self.n_heads * self.head_dim)
+        return (self.tables[self._rows].contiguous(), full(end), full(start), q_start, full(ntok),
+                ntok)
 
     # ---- linear back ends ---------------------------------------------------------------------
 
@@ -207,21 +213,20 @@ class DecodeRunner:
         """normed (1, nseq*ntok, hidden), sequences contiguous, every sequence at positions
         [start, start + ntok). Writes K/V there and attends causally over [0, end). The
         positions come in as a host int, so a step captures into a graph."""
-        from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
-
         q, k, v = self._qkv(i, normed)
-        q = q.reshape(nseq, ntok, self.n_heads, self.head_dim).transpose(1, 2)
-        k = k.reshape(nseq, ntok, self.n_kv, self.head_dim).transpose(1, 2)
-        v = v.reshape(nseq, ntok, self.n_kv, self.head_dim).transpose(1, 2)
-        cos, sin = rope
-        q, k = apply_rotary_pos_emb(q, k, cos, sin)
         end = start + ntok
-        self.k_cache[i][self._rows, :, start:end] = k
-        self.v_cache[i][self._rows, :, start:end] = v
+        rows = self._rows
+        pool = None
         if self.k_pool is not None:
-            self._write_pool(i, k, v, start, end, self._rows)
+            pool = (self.k_pool[i], self.v_pool[i], self.tables[rows])
+        if self._fused and nseq * ntok <= 65535:
+            q = ops.rope_kv(q[0], k[0], v[0], *rope, self.n_heads, self.n_kv, nseq, start,
+                            (self.k_cache[i][rows], self.v_cache[i][rows]), pool)
+        else:
+            q = self._rope_kv_torch(i, q, k, v, rope, start, nseq, ntok)
         if self.attention == "paged":
-            return self._o(i, self._attend_paged(i, q, start, end, nseq, ntok))
+            return self._o(i, self._attend_paged(i, q))
+        q = q.reshape(nseq, ntok, self.n_heads, self.head_dim).transpose(1, 2)
         keys = self.k_cache[i][self._rows, :, :end].float()
         vals = self.v_cache[i][self._rows, :, :end].float()
         rep = self.n_heads // self.n_kv
@@ -236,6 +241,44 @@ class DecodeRunner:
         out = out.to(torch.bfloat16).transpose(1, 2).reshape(1, nseq * ntok, -1)
         return self._o(i, out)
 
+    def _rope_kv_torch(self, i: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rope,
+                       start: int, nseq: int, ntok: int) -> torch.Tensor:
+        """What `ops.rope_kv` does, with the reference's own eager operations (devices and dtypes
+        the kernel does not take)."""
+        from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
+
+        q = q.reshape(nseq, ntok, self.n_heads, self.head_dim).transpose(1, 2)
+        k = k.reshape(nseq, ntok, self.n_kv, self.head_dim).transpose(1, 2)
+        v = v.reshape(nseq, ntok, self.n_kv, self.head_dim).transpose(1, 2)
+        cos, sin = (t.reshape(nseq, ntok, -1) for t in rope)
+        q, k = apply_rotary_pos_emb(q, k, cos, sin)
+        end = start + ntok
+        self.k_cache[i][self._rows, :, start:end] = k
+        self.v_cache[i][self._rows, :, start:end] = v
+        if self.k_pool is not None:
+            self._write_pool(i, k, v, start, end, self._rows)
+        return q.transpose(1, 2).reshape(nseq * ntok, self.n_heads, self.head_dim)
+
+    def _add_norm(self, norm: nn.Module, x: torch.Tensor, residual: torch.Tensor | None):
+        """(x + residual, norm(x + residual)), as one kernel where it can be."""
+        if self._fused:
+            return ops.add_rmsnorm(x, residual, norm.weight, norm.variance_epsilon)
+        hidden = x if residual is None else residual + x
+        return hidden, norm(hidden)
+
+    def _fusable(self) -> bool:
+        """Whether the rotary embedding, the K/V writes and the norms of this model run as the fused
+        kernels: bf16 on the GPU, plain LlamaRMSNorms without hooks, a head and a row size they
+        take."""
+        model = self.model.model
+        norms = [model.norm, *(n for layer in self.layers
+                               for n in (layer.input_layernorm, layer.post_attention_layernorm))]
+        return (self.k_cache[0].is_cuda and self.head_dim % 16 == 0 and self.head_dim <= 1024
+                and norms[0].weight.shape[0] % 8 == 0
+                and norms[0].weight.shape[0] <= _lib.NORM_MAX_K
+                and all(type(n).__name__ == "LlamaRMSNorm" and n.weight.dtype == torch.bfloat16
+                        and not (n._forward_hooks or n._forward_pre_hooks) for n in norms))
+
     @torch.no_grad()
     def forward(self, tokens: torch.Tensor, start: int, rows: slice | None = None) -> torch.Tensor:
         """tokens (nseq, ntok) of sequences `rows` (default: all) at positions [start,
@@ -247,12 +290,18 @@ class DecodeRunner:
         pos = torch.arange(start, start + ntok, device=tokens.device).repeat(nseq, 1)
         hidden = model.embed_tokens(ids)
         cos, sin = model.rotary_emb(hidden, pos.reshape(1, -1))
-        rope = (cos.reshape(nseq, ntok, -1), sin.reshape(nseq, ntok, -1))
+        self._fused = self._fusable() and hidden.dtype == cos.dtype == torch.bfloat16
+        rope = (cos[0], sin[0])
+        if self.attention == "paged":
+            self._plan = self._paged_plan(start, start + ntok, nseq, ntok)
+        norms = [layer.input_layernorm for layer in self.layers] + [model.norm]
+        hidden, normed = self._add_norm(norms[0], hidden, None)
         for i, layer in enumerate(self.layers):
-            hidden = hidden + self._attend(i, layer.input_layernorm(hidden), rope, start, nseq,
-                                           ntok)
-            hidden = hidden + self._mlp(i, layer.post_attention_layernorm(hidden))
-        return model.norm(hidden)
+            out = self._attend(i, normed, rope, start, nseq, ntok)
+            hidden, normed = self._add_norm(layer.post_attention_layernorm, out, hidden)
+            hidden, normed = self._add_norm(norms[i + 1], self._mlp(i, normed), hidden)
+        self._plan = None  # its tensors live as long as the call
+        return normed
 
     @torch.no_grad()
     def prefill(self, tokens: torch.Tensor, chunk: int = 8) -> None:

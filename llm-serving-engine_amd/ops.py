@@ -17,6 +17,7 @@ import torch
 from . import _lib
 
 __all__ = [
+    "add_rmsnorm",
     "bf16_decode_linear",
     "pack_bf16_weight",
     "packed_bf16_shape",
@@ -29,6 +30,7 @@ __all__ = [
     "quantize_act_per_token",
     "quantize_weight_per_channel",
     "rmsnorm_quantize",
+    "rope_kv",
     "unpack_glu",
     "unpack_weight",
     "w8a8_gemm",
@@ -454,6 +456,96 @@ def rmsnorm_quantize(
         "lse_rmsnorm_quantize",
     )
     return xq, sx, normed
+
+
+def add_rmsnorm(
+    x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor, eps: float,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """(s, LlamaRMSNorm(s)) with s = x + residual (x itself when residual is None) in one kernel:
+    x and residual (..., K) bf16, weight (K,) bf16, K <= `_lib.NORM_MAX_K`."""
+    dev = _on_gpu(x, weight) if residual is None else _on_gpu(x, weight, residual)
+    k = x.shape[-1]
+    _require(x.dtype == weight.dtype == torch.bfloat16 and weight.shape == (k,),
+             f"RMSNorm takes bf16 x and weight ({k},)")
+    x2 = _rows(x, k)
+    m = x2.shape[0]
+    y = torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
+    if residual is None:
+        r2, s = None, x
+    else:
+        _require(residual.dtype == torch.bfloat16 and residual.shape == x.shape,
+                 "the residual must be bf16 and of x's shape")
+        r2, s = _rows(residual, k), torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
+    w = weight.contiguous()
+    _lib.check(
+        _lib.library().lse_add_rmsnorm(
+            x2.data_ptr(), x2.stride(0) if m > 1 else k,
+            r2.data_ptr() if r2 is not None else None,
+            r2.stride(0) if r2 is not None and m > 1 else k, w.data_ptr(), float(eps),
+            s.data_ptr() if r2 is not None else None, y.data_ptr(), m, k, _stream(dev)),
+        "lse_add_rmsnorm",
+    )
+    return s, y
+
+
+def rope_kv(
+    q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+    n_heads: int, n_kv: int, sequences: int, start: int,
+    cache: tuple[torch.Tensor, torch.Tensor] | None = None,
+    pool: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
+) -> torch.Tensor:
+    """Rotates one layer's new q and k (`apply_rotary_pos_emb`, the same bits) and writes k and v at
+    positions [start, start + tokens / sequences) of every sequence, in one kernel.
+
+    q (..., n_heads D), k and v (..., n_kv D): bf16, rows of consecutive sequences' tokens, the last
+    dim contiguous. cos, sin (tokens, D) bf16. cache: (k, v) of (sequences, n_kv, capacity, D).
+    pool: (k, v, table) of (blocks, block_size, n_kv, D) and int32 (sequences, blocks). Returns the
+    rotated q as (tokens, n_heads, D)."""
+    dev = _on_gpu(q, k, v, cos, sin)
+    d = cos.shape[-1]
+    rows = []
+    for name, t, width in (("q", q, n_heads * d), ("k", k, n_kv * d), ("v", v, n_kv * d),
+                           ("cos", cos, d), ("sin", sin, d)):
+        _require(t.dtype == torch.bfloat16, f"{name} must be bf16, got {t.dtype}")
+        rows.append(_rows(t, width))
+    tokens = rows[0].shape[0]
+    _require(all(t.shape[0] == tokens for t in rows) and tokens % max(1, sequences) == 0,
+             "q, k, v, cos and sin need one row per token of every sequence")
+    ntok = tokens // max(1, sequences)
+    if rows[4].stride(0) != rows[3].stride(0):
+        rows[3], rows[4] = rows[3].contiguous(), rows[4].contiguous()
+    out = torch.empty((tokens, n_heads, d), dtype=torch.bfloat16, device=dev)
+    cache_args, pool_args = [None, None, 0, 0, 0], [None, None, 0, 0, 0, None, 0, 1]
+    if cache is not None:
+        kc, vc = cache
+        _on_gpu(q, kc, vc)
+        _require(kc.dtype == vc.dtype == torch.bfloat16 and kc.shape == vc.shape
+                 and kc.stride() == vc.stride() and kc.stride(3) == 1
+                 and kc.shape[:2] == (sequences, n_kv) and kc.shape[3] == d
+                 and kc.shape[2] >= start + ntok,
+                 f"cache must be two bf16 ({sequences}, {n_kv}, >= {start + ntok}, {d}) tensors")
+        cache_args = [kc.data_ptr(), vc.data_ptr(), *kc.stride()[:3]]
+    if pool is not None:
+        kp, vp, table = pool
+        _on_gpu(q, kp, vp, table)
+        _require(kp.dtype == vp.dtype == torch.bfloat16 and kp.shape == vp.shape
+                 and kp.stride() == vp.stride() and kp.stride(3) == 1
+                 and kp.shape[2:] == (n_kv, d), f"pool must be two bf16 (*, *, {n_kv}, {d}) tensors")
+        _require(table.dtype == torch.int32 and table.dim() == 2 and table.stride(1) == 1
+                 and table.shape[0] == sequences
+                 and table.shape[1] * kp.shape[1] >= start + ntok,
+                 f"table must be int32, {sequences} rows covering {start + ntok} positions")
+        pool_args = [kp.data_ptr(), vp.data_ptr(), *kp.stride()[:3], table.data_ptr(),
+                     table.stride(0), kp.shape[1]]
+    ld = [t.stride(0) if tokens > 1 else t.shape[1] for t in rows]
+    _lib.check(
+        _lib.library().lse_rope_kv(
+            rows[0].data_ptr(), ld[0], rows[1].data_ptr(), ld[1], rows[2].data_ptr(), ld[2],
+            rows[3].data_ptr(), rows[4].data_ptr(), ld[3], out.data_ptr(), *cache_args, *pool_args,
+            n_heads, n_kv, d, sequences, ntok, start, _stream(dev)),
+        "lse_rope_kv",
+    )
+    return out
 
 
 def packed_bf16_shape(n: int, k: int) -> tuple[int, int, int]:

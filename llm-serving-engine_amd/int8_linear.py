@@ -112,11 +112,16 @@ class Int8Linear(nn.Module):
 
     def forward(self, x: torch.Tensor | QuantizedRows) -> torch.Tensor:
         group = self.__dict__.get("_qkv_group")
+        buffers = self._buffers
+        try:  # nn.Module's own attribute lookup costs half a microsecond each
+            qweight, scales, bias = buffers["qweight"], buffers["scales"], buffers["bias"]
+        except KeyError:  # replaced by something that is no buffer
+            qweight, scales, bias = self.qweight, self.scales, self.bias
         if group is not None:
             y = group.columns(self, x)
         else:
-            y = _int8_product(self.mode, x, self.qweight, self.scales, self.out_features)
-        return y if self.bias is None else y + self.bias
+            y = _int8_product(self.mode, x, qweight, scales, self.out_features)
+        return y if bias is None else y + bias
 
     def extra_repr(self) -> str:
         return (

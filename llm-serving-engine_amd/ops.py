@@ -44,8 +44,17 @@ __all__ = [
 ]
 
 
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+# A decode call's kernel runs 5 to 10 us, so the checks before it are written for their cost on the
+# host: plain conditions with the message built only to raise it, device indices and raw stream
+# handles instead of device and stream objects, and no view of the input or the output where their
+# memory already has the rows the kernel takes. An eager `Int8Linear` call of one row went from 18.2
+# to about 11 us a call.
+
+
+def _stream(device: torch.device | int) -> int:
+    if not isinstance(device, int):
+        device = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -53,12 +62,15 @@ def _require(cond: bool, msg: str) -> None:
         raise RuntimeError(msg)
 
 
-def _on_gpu(*tensors: torch.Tensor) -> torch.device:
-    dev = tensors[0].device
-    _require(dev.type == "cuda", f"int8 kernels need a CUDA (HIP) device, got {dev}")
-    for t in tensors[1:]:
-        _require(t.device == dev, f"tensors on different devices: {dev} and {t.device}")
-    return dev
+def _on_gpu(first: torch.Tensor, *others: torch.Tensor) -> int:
+    """The index of the GPU all of the tensors are on."""
+    if not first.is_cuda:
+        raise RuntimeError(f"int8 kernels need a CUDA (HIP) device, got {first.device}")
+    index = first.get_device()
+    for t in others:
+        if not t.is_cuda or t.get_device() != index:
+            raise RuntimeError(f"tensors on different devices: {first.device} and {t.device}")
+    return index
 
 
 def _rows(x: torch.Tensor, k: int) -> torch.Tensor:
@@ -69,6 +81,18 @@ def _rows(x: torch.Tensor, k: int) -> torch.Tensor:
     if x2.stride(-1) != 1 or strided_rows or x2.data_ptr() % 16:
         x2 = x2.contiguous()
     return x2
+
+
+def _row_args(x: torch.Tensor, k: int) -> tuple[torch.Tensor, int, int, int]:
+    """(owner, address, row stride, rows) of x (..., K) as `_rows` gives them; `owner` is to be
+    kept until the kernel is enqueued."""
+    if k and x.is_contiguous() and x.shape[-1] == k:
+        at = x.data_ptr()
+        if at % 16 == 0:
+            return x, at, k, x.numel() // k
+    x2 = _rows(x, k)
+    m = x2.shape[0]
+    return x2, x2.data_ptr(), x2.stride(0) if m > 1 else k, m
 
 
 # ---- packed weights --------------------------------------------------------------------------
@@ -125,12 +149,14 @@ def unpack_glu(qp: torch.Tensor, i: int, k: int) -> torch.Tensor:
     return torch.cat([gate, up]).contiguous()
 
 
-def workspace(mode: int, m: int, n: int, k: int, dev: torch.device) -> torch.Tensor | None:
+def workspace(mode: int, m: int, n: int, k: int,
+              dev: torch.device | int) -> torch.Tensor | None:
     """The workspace one GEMM call needs (deep decode shapes and 65..256 tokens over a narrow
     weight add partial sums of K ranges in a second pass), or None. Allocated with torch.empty,
     so graph-pool owned under capture; the caller keeps it alive until the call is enqueued."""
     nbytes = _lib.library().lse_workspace_bytes(mode, m, n, k)
-    _require(nbytes >= 0, f"lse_workspace_bytes rejected (M, N, K) = ({m}, {n}, {k})")
+    if nbytes < 0:
+        raise RuntimeError(f"lse_workspace_bytes rejected (M, N, K) = ({m}, {n}, {k})")
     return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
 
 
@@ -139,16 +165,29 @@ def _ws_args(ws: torch.Tensor | None) -> tuple[int | None, int]:
 
 
 def _check_packed(qp: torch.Tensor, n: int, k: int, glu: bool = False) -> None:
-    _require(qp.dtype == torch.int8 and qp.is_contiguous(), "packed weight must be contiguous int8")
+    if qp.dtype is not torch.int8 or not qp.is_contiguous():
+        raise RuntimeError("packed weight must be contiguous int8")
     want = packed_glu_shape(n, k) if glu else packed_shape(n, k)
-    what = "(I, K)" if glu else "(N, K)"
-    _require(tuple(qp.shape) == want,
-             f"packed weight has shape {tuple(qp.shape)}, {what} = ({n}, {k}) needs {want}")
+    if qp.shape != want:
+        what = "(I, K)" if glu else "(N, K)"
+        raise RuntimeError(f"packed weight has shape {tuple(qp.shape)}, {what} = ({n}, {k}) needs "
+                           f"{want}")
+
+
+def _check_bf16(x: torch.Tensor, what: str) -> None:
+    if x.dtype is not torch.bfloat16:
+        raise RuntimeError(f"{what} expects bf16 activations, got {x.dtype}")
+
+
+def _channel_scales(scales: torch.Tensor) -> int:
+    if scales.dtype is not torch.float32 or scales.dim() != 1:
+        raise RuntimeError("scales must be fp32 (N,)")
+    return scales.shape[0]
 
 
 def _glu_scales(scales: torch.Tensor) -> int:
-    _require(scales.dtype == torch.float32 and scales.dim() == 1 and scales.shape[0] % 2 == 0,
-             "gate/up scales must be fp32 (2I,) [gate; up]")
+    if scales.dtype is not torch.float32 or scales.dim() != 1 or scales.shape[0] % 2:
+        raise RuntimeError("gate/up scales must be fp32 (2I,) [gate; up]")
     return scales.shape[0] // 2
 
 
@@ -185,23 +224,21 @@ def w8a16_linear(
     """y = bf16(s[n] * sum_k x[..., k] q[n, k]) for x (..., K) bf16 → y (..., N) bf16, with the
     weight q given packed (`pack_weight`)."""
     dev = _on_gpu(x, qp, scales)
-    _require(x.dtype == torch.bfloat16, f"W8A16 expects bf16 activations, got {x.dtype}")
-    _require(scales.dtype == torch.float32 and scales.dim() == 1, "scales must be fp32 (N,)")
-    n, k = scales.shape[0], x.shape[-1]
+    _check_bf16(x, "W8A16")
+    n, lead = _channel_scales(scales), x.shape
+    k = lead[-1]
     _check_packed(qp, n, k)
-    x2 = _rows(x, k)
-    m = x2.shape[0]
-    y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
-    ldx = x2.stride(0) if m > 1 else k
+    owner, at, ldx, m = _row_args(x, k)
+    y = torch.empty((*lead[:-1], n), dtype=torch.bfloat16, device=dev)
     ws = workspace(_lib.MODE_W8A16, m, n, k, dev)
     _lib.check(
         _lib.library().lse_w8a16_gemm_algo(
-            x2.data_ptr(), ldx, qp.data_ptr(), scales.data_ptr(), y.data_ptr(), n,
-            m, n, k, algo, *_ws_args(ws), _stream(dev),
+            at, ldx, qp.data_ptr(), scales.data_ptr(), y.data_ptr(), n, m, n, k, algo,
+            *_ws_args(ws), _stream(dev),
         ),
         "lse_w8a16_gemm",
     )
-    return y.view(*x.shape[:-1], n)
+    return y
 
 
 def w8a16_linear_noalloc(x: torch.Tensor, qp: torch.Tensor, scales: torch.Tensor,
@@ -229,20 +266,27 @@ def w8a16_linear_noalloc(x: torch.Tensor, qp: torch.Tensor, scales: torch.Tensor
 def quantize_act_per_token(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """x (..., K) bf16 → (xq (rows, K) int8, sx (rows,) fp32), per-row symmetric int8."""
     dev = _on_gpu(x)
-    _require(x.dtype == torch.bfloat16, f"W8A8 expects bf16 activations, got {x.dtype}")
+    _check_bf16(x, "W8A8")
     k = x.shape[-1]
-    x2 = _rows(x, k)
-    m = x2.shape[0]
+    owner, at, ldx, m = _row_args(x, k)
     xq = torch.empty((m, k), dtype=torch.int8, device=dev)
     sx = torch.empty((m,), dtype=torch.float32, device=dev)
-    ldx = x2.stride(0) if m > 1 else k
     _lib.check(
         _lib.library().lse_quantize_act_per_token(
-            x2.data_ptr(), ldx, xq.data_ptr(), sx.data_ptr(), m, k, _stream(dev)
+            at, ldx, xq.data_ptr(), sx.data_ptr(), m, k, _stream(dev)
         ),
         "lse_quantize_act_per_token",
     )
     return xq, sx
+
+
+def _quantized_rows(xq: torch.Tensor, sx: torch.Tensor, msg: str) -> tuple[int, int]:
+    if xq.dim() != 2 or xq.dtype is not torch.int8 or not xq.is_contiguous():
+        raise RuntimeError(msg)
+    m, k = xq.shape
+    if sx.dtype is not torch.float32 or sx.shape != (m,):
+        raise RuntimeError("sx must be fp32 (M,)")
+    return m, k
 
 
 def w8a8_gemm(
@@ -256,12 +300,8 @@ def w8a8_gemm(
     """(y (M, N) bf16 or None, acc (M, N) int32 or None) from quantized operands; the weight q
     is given packed."""
     dev = _on_gpu(xq, sx, qp, scales)
-    _require(scales.dtype == torch.float32 and scales.dim() == 1, "scales must be fp32 (N,)")
-    n = scales.shape[0]
-    _require(xq.dim() == 2, "xq must be (M, K) int8")
-    m, k = xq.shape
-    _require(xq.dtype == torch.int8 and xq.is_contiguous(), "xq must be (M, K) int8")
-    _require(sx.dtype == torch.float32 and sx.shape == (m,), "sx must be fp32 (M,)")
+    n = _channel_scales(scales)
+    m, k = _quantized_rows(xq, sx, "xq must be (M, K) int8")
     _check_packed(qp, n, k)
     y = torch.empty((m, n), dtype=torch.bfloat16, device=dev) if want_y else None
     acc = torch.empty((m, n), dtype=torch.int32, device=dev) if want_acc else None
@@ -299,16 +339,15 @@ def w8a8_linear(x: torch.Tensor, qp: torch.Tensor, scales: torch.Tensor,
         one_launch = m * k <= ONE_LAUNCH_W8A8_MAX_ELEMS
     if m and one_launch and lib.lse_w8a8_linear_supported(m, k):
         dev = _on_gpu(x, qp, scales)
-        _require(x.dtype == torch.bfloat16, f"W8A8 expects bf16 activations, got {x.dtype}")
-        _require(scales.dtype == torch.float32 and scales.dim() == 1, "scales must be fp32 (N,)")
+        _check_bf16(x, "W8A8")
+        _channel_scales(scales)
         _check_packed(qp, n, k)
-        x2 = _rows(x, k)
+        owner, at, ldx, _ = _row_args(x, k)
         y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
         acc = torch.empty((m, n), dtype=torch.int32, device=dev) if want_acc else None
-        ldx = x2.stride(0) if m > 1 else k
         _lib.check(
             lib.lse_w8a8_linear(
-                x2.data_ptr(), ldx, qp.data_ptr(), scales.data_ptr(), y.data_ptr(), n,
+                at, ldx, qp.data_ptr(), scales.data_ptr(), y.data_ptr(), n,
                 acc.data_ptr() if acc is not None else None, m, n, k, _stream(dev),
             ),
             "lse_w8a8_linear",
@@ -330,21 +369,19 @@ def w8a16_glu(
     W8A16 products of x with the gate and up weights (`pack_glu` layout, scales (2I,) [gate;
     up]); one kernel, one rounding."""
     dev = _on_gpu(x, qp, scales)
-    _require(x.dtype == torch.bfloat16, f"W8A16 expects bf16 activations, got {x.dtype}")
-    i, k = _glu_scales(scales), x.shape[-1]
+    _check_bf16(x, "W8A16")
+    i, lead = _glu_scales(scales), x.shape
+    k = lead[-1]
     _check_packed(qp, i, k, glu=True)
-    x2 = _rows(x, k)
-    m = x2.shape[0]
-    h = torch.empty((m, i), dtype=torch.bfloat16, device=dev)
-    ldx = x2.stride(0) if m > 1 else k
+    owner, at, ldx, m = _row_args(x, k)
+    h = torch.empty((*lead[:-1], i), dtype=torch.bfloat16, device=dev)
     _lib.check(
         _lib.library().lse_w8a16_glu(
-            x2.data_ptr(), ldx, qp.data_ptr(), scales.data_ptr(), h.data_ptr(), i, m, i, k, algo,
-            _stream(dev),
+            at, ldx, qp.data_ptr(), scales.data_ptr(), h.data_ptr(), i, m, i, k, algo, _stream(dev),
         ),
         "lse_w8a16_glu",
     )
-    return h.view(*x.shape[:-1], i)
+    return h
 
 
 def w8a8_glu(x: torch.Tensor, qp: torch.Tensor, scales: torch.Tensor) -> torch.Tensor:
@@ -360,10 +397,7 @@ def w8a8_glu_quantized(xq: torch.Tensor, sx: torch.Tensor, qp: torch.Tensor,
     """`w8a8_glu` from already quantized rows: xq (M, K) int8, sx (M,) fp32 → h (M, I) bf16."""
     dev = _on_gpu(xq, sx, qp, scales)
     i = _glu_scales(scales)
-    _require(xq.dim() == 2 and xq.dtype == torch.int8 and xq.is_contiguous(),
-             "xq must be contiguous (M, K) int8")
-    m, k = xq.shape
-    _require(sx.dtype == torch.float32 and sx.shape == (m,), "sx must be fp32 (M,)")
+    m, k = _quantized_rows(xq, sx, "xq must be contiguous (M, K) int8")
     _check_packed(qp, i, k, glu=True)
     h = torch.empty((m, i), dtype=torch.bfloat16, device=dev)
     _lib.check(
@@ -390,31 +424,36 @@ def paged_attention_forward(
     q_start, q_len (entries,): int32 on the device. max_q_len >= every q_len. Returns o like q.
     Softmax scale 1/sqrt(D). D = 128 and 1 <= H / H_KV <= 16 (24 query heads over 8 K/V
     heads included)."""
-    dev = _on_gpu(q, k_pool, v_pool, block_table, context_len, query_offset, q_start, q_len)
-    _require(q.dim() == 3 and k_pool.dim() == 4 and v_pool.shape == k_pool.shape,
-             "q must be (H, T, D), k_pool/v_pool (num_blocks, block_size, H_KV, D)")
-    _require(q.dtype == k_pool.dtype == v_pool.dtype == torch.bfloat16,
-             f"paged attention runs on bf16 q/k/v, got {q.dtype}, {k_pool.dtype}, {v_pool.dtype}")
-    for name, t in (("block_table", block_table), ("context_len", context_len),
-                    ("query_offset", query_offset), ("q_start", q_start), ("q_len", q_len)):
-        _require(t.dtype == torch.int32, f"{name} must be int32, got {t.dtype}")
-    _require(block_table.dim() == 2 and block_table.stride(1) == 1, "block_table must be (E, B) "
-             "with unit column stride")
+    entry = (context_len, query_offset, q_start, q_len)
+    dev = _on_gpu(q, k_pool, v_pool, block_table, *entry)
+    if q.dim() != 3 or k_pool.dim() != 4 or v_pool.shape != k_pool.shape:
+        raise RuntimeError("q must be (H, T, D), k_pool/v_pool (num_blocks, block_size, H_KV, D)")
+    bf16 = torch.bfloat16
+    if q.dtype is not bf16 or k_pool.dtype is not bf16 or v_pool.dtype is not bf16:
+        raise RuntimeError(f"paged attention runs on bf16 q/k/v, got {q.dtype}, {k_pool.dtype}, "
+                           f"{v_pool.dtype}")
+    names = ("context_len", "query_offset", "q_start", "q_len")
+    for name, t in zip(("block_table", *names), (block_table, *entry)):
+        if t.dtype is not torch.int32:
+            raise RuntimeError(f"{name} must be int32, got {t.dtype}")
+    if block_table.dim() != 2 or block_table.stride(1) != 1:
+        raise RuntimeError("block_table must be (E, B) with unit column stride")
     entries = block_table.shape[0]
-    for name, t in (("context_len", context_len), ("query_offset", query_offset),
-                    ("q_start", q_start), ("q_len", q_len)):
-        _require(t.dim() == 1 and t.shape[0] == entries and t.stride(0) == 1,
-                 f"{name} must be a contiguous ({entries},) tensor")
+    for name, t in zip(names, entry):
+        if t.shape != (entries,) or t.stride(0) != 1:
+            raise RuntimeError(f"{name} must be a contiguous ({entries},) tensor")
     h, _tokens, d = q.shape
     _, bs, h_kv, dk = k_pool.shape
-    _require(dk == d and bs == block_size, "pool shape does not match q / block_size")
-    _require(q.stride(2) == 1 and k_pool.stride(3) == 1 and v_pool.stride() == k_pool.stride(),
-             "head dim must be contiguous and k_pool/v_pool must share strides")
+    if dk != d or bs != block_size:
+        raise RuntimeError("pool shape does not match q / block_size")
+    if q.stride(2) != 1 or k_pool.stride(3) != 1 or v_pool.stride() != k_pool.stride():
+        raise RuntimeError("head dim must be contiguous and k_pool/v_pool must share strides")
     o = torch.empty_like(q)
     lib = _lib.library()
     nbytes = lib.lse_paged_attention_workspace_bytes(entries, h, h_kv, d, max_q_len,
                                                      block_table.shape[1], block_size)
-    _require(nbytes >= 0, f"unsupported attention shape: H={h} H_KV={h_kv} D={d}")
+    if nbytes < 0:
+        raise RuntimeError(f"unsupported attention shape: H={h} H_KV={h_kv} D={d}")
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
     _lib.check(
         lib.lse_paged_attention(
@@ -437,19 +476,20 @@ def rmsnorm_quantize(
     bf16 output in one kernel: x (..., K) bf16, weight (K,) bf16 → (xq (rows, K) int8, sx (rows,)
     fp32, normed (rows, K) bf16 or None)."""
     dev = _on_gpu(x, weight)
-    _require(x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16,
-             f"RMSNorm-quantize takes bf16 x and weight, got {x.dtype}, {weight.dtype}")
+    if x.dtype is not torch.bfloat16 or weight.dtype is not torch.bfloat16:
+        raise RuntimeError(
+            f"RMSNorm-quantize takes bf16 x and weight, got {x.dtype}, {weight.dtype}")
     k = x.shape[-1]
-    _require(weight.shape == (k,), f"weight must be ({k},), got {tuple(weight.shape)}")
-    x2 = _rows(x, k)
-    m = x2.shape[0]
+    if weight.shape != (k,):
+        raise RuntimeError(f"weight must be ({k},), got {tuple(weight.shape)}")
+    owner, at, ldx, m = _row_args(x, k)
     w = weight.contiguous()
     xq = torch.empty((m, k), dtype=torch.int8, device=dev)
     sx = torch.empty((m,), dtype=torch.float32, device=dev)
     normed = torch.empty((m, k), dtype=torch.bfloat16, device=dev) if want_normed else None
     _lib.check(
         _lib.library().lse_rmsnorm_quantize(
-            x2.data_ptr(), x2.stride(0) if m > 1 else k, w.data_ptr(), float(eps),
+            at, ldx, w.data_ptr(), float(eps),
             xq.data_ptr(), sx.data_ptr(), normed.data_ptr() if normed is not None else None, m,
             k, _stream(dev),
         ),
@@ -579,18 +619,18 @@ def bf16_decode_linear(x: torch.Tensor, wp: torch.Tensor, n: int) -> torch.Tenso
     bf16; fp32 accumulation. Built for decode batches (the decode kernel up to 16 rows, bf16
     tiles of the tiled kernel above), correct for any number of rows."""
     dev = _on_gpu(x, wp)
-    _require(x.dtype == torch.bfloat16, f"expects bf16 activations, got {x.dtype}")
-    k = x.shape[-1]
-    _require(wp.dtype == torch.bfloat16 and tuple(wp.shape) == packed_bf16_shape(n, k),
-             f"packed weight has shape {tuple(wp.shape)}, (N, K) = ({n}, {k}) needs "
-             f"{packed_bf16_shape(n, k)}")
-    x2 = _rows(x, k)
-    m = x2.shape[0]
-    y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    if x.dtype is not torch.bfloat16:
+        raise RuntimeError(f"expects bf16 activations, got {x.dtype}")
+    lead = x.shape
+    k = lead[-1]
+    if wp.dtype is not torch.bfloat16 or wp.shape != packed_bf16_shape(n, k):
+        raise RuntimeError(f"packed weight has shape {tuple(wp.shape)}, (N, K) = ({n}, {k}) needs "
+                           f"{packed_bf16_shape(n, k)}")
+    owner, at, ldx, m = _row_args(x, k)
+    y = torch.empty((*lead[:-1], n), dtype=torch.bfloat16, device=dev)
     _lib.check(
-        _lib.library().lse_bf16_decode_gemm(x2.data_ptr(), x2.stride(0) if m > 1 else k,
-                                            wp.data_ptr(), y.data_ptr(), n, m, n, k,
+        _lib.library().lse_bf16_decode_gemm(at, ldx, wp.data_ptr(), y.data_ptr(), n, m, n, k,
                                             _stream(dev)),
         "lse_bf16_decode_gemm",
     )
-    return y.view(*x.shape[:-1], n)
+    return y

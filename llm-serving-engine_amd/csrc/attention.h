@@ -25,6 +25,8 @@ struct PagedAttnArgs {
   int tq;            // query tokens per tile: floor(16 / G)
   int qtiles;        // ceil(max_q_len / tq)
   int parts;         // 1: a workgroup folds every chunk of its item; > 1: one chunk per workgroup
+  int sorted;        // entries are taken in descending order of context length...
+  int first_round;   // ...and, where > 0, those from this rank on in ascending order
   float scale_log2;  // softmax scale x log2(e): scores are kept in the base-2 domain
   float* ws_o;       // parts > 1: chunk states' O [parts][entries][H][max_q_len][D], fp32
   float* ws_ml;      // parts > 1: chunk states' max and sum [parts][entries][H][max_q_len][2]

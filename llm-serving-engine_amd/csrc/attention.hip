@@ -92,6 +92,26 @@ __device__ __forceinline__ uint4 attn_out8(float L, const float (&O)[8]) {
   return out;
 }
 
+// The entry of rank `slot` by context length, longest first (entries without work for this kernel
+// last; at most 64 entries, one per lane). Workgroups are dispatched in order, so long ones start first
+// and short ones fill the gaps. With up to two workgroups per CU all start at once and a CU's two
+// share its bandwidth: ranks past the first round run backwards (a.first_round), so that the
+// longest entries share their CU with the shortest. Every wave ranks for itself, in registers.
+__device__ __forceinline__ int attn_sorted_entry(const PagedAttnArgs& a, int slot) {
+  const int lane = threadIdx.x & 63;
+  int key = -1;  // longer first, then the lower index
+  if (lane < a.entries) {
+    const int qlen = a.q_len[lane], ctx = a.context_len[lane];
+    const bool none = qlen == 0 || (a.tiled && attn_is_long((int64_t)qlen * a.G, ctx));
+    key = ((none ? 0 : 1 + min(max(ctx, 0), (1 << 24) - 1)) << 6) + 63 - lane;
+  }
+  int rank = 0;
+#pragma unroll
+  for (int j = 0; j < 64; ++j) rank += __builtin_amdgcn_readlane(key, j) > key;
+  if (a.first_round > 0 && slot >= a.first_round) slot = a.first_round + a.entries - 1 - slot;
+  return __ffsll(__ballot(rank == slot && lane < a.entries)) - 1;
+}
+
 // NT: K and V stream with the nt cache policy; used when each K/V row is read by one workgroup
 // only (one query tile: decode). POW2: block_size is a power of two (a shift finds a key's block).
 template <int D, bool NT, bool POW2>
@@ -120,11 +140,12 @@ paged_attn_kernel(PagedAttnArgs a) {
   int b = blockIdx.x;
   const int kvh = b % a.HKV;
   b /= a.HKV;
-  const int e = b % a.entries;
+  int e = b % a.entries;
   b /= a.entries;
   const int part = b % a.parts;
   const int qt = b / a.parts;
   const int G = a.G, TQ = a.tq;
+  if (a.sorted && qt == 0) e = attn_sorted_entry(a, e);
   const int qlen = a.q_len[e];
   if (qt * TQ >= qlen) return;
   const int ctx = a.context_len[e];
@@ -474,6 +495,12 @@ int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const 
     if (int st = launch_attn_tile(a, attn_cus(), stream)) return st;
     a.max_q_len = (int)pl.short_q;
   }
+  // Measured on MI355X: 64 decode rows over 8 K/V heads, contexts 256 to 2048 (300 MB of K and V),
+  // 74.6 us in the given order, 58.9 sorted; 40 rows beside a 735-token chunk 98 and 88; 64 rows of one
+  // context the same within 0.2 us. Split launches (few items) start everything at once anyway.
+  const int64_t cus = attn_cus(), items = (int64_t)a.entries * a.HKV;
+  a.sorted = a.parts == 1 && a.entries > 1 && a.entries <= 64;
+  a.first_round = items > cus && items <= 2 * cus && cus % a.HKV == 0 ? (int)(cus / a.HKV) : 0;
   void* args[] = {&a};
   const bool pow2 = a.bs_shift >= 0;
   const void* fn =

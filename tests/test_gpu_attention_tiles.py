@@ -83,3 +83,19 @@ def test_more_entries_than_one_launch_holds(pkg, dev):
     entries = [(17 if e % 100 == 0 or e > 1026 else 1, 0, 17 if e % 100 == 0 or e > 1026 else 1)
                for e in range(1030)]
     _check(pkg, dev, _case(600, entries, h=16, h_kv=1), "1030 entries")
+
+
+@pytest.mark.parametrize("entries", [2, 33, 63, 64, 65])
+def test_entries_in_order_of_length(pkg, dev, entries):
+    """Decode rows of different and equal contexts, with padding rows (q_len 0), on both sides of
+    the entry counts whose workgroups are ordered by length and paired on a CU."""
+    rng = np.random.default_rng(entries)
+    ctx = rng.integers(1, 90, entries)
+    ctx[::3] = 40
+    c = _case(700 + entries, [(1, int(n) - 1, int(n)) for n in ctx], h=8, h_kv=8)
+    base = _check(pkg, dev, c, f"{entries} entries")
+    pad = dict(c, ql=c["ql"].copy(), ctx=c["ctx"].copy())
+    pad["ql"][1::7] = pad["ctx"][1::7] = 0
+    o = _run(pkg, dev, pad)
+    keep = pad["ql"] > 0
+    np.testing.assert_array_equal(o[:, keep], base[:, keep])

@@ -94,9 +94,11 @@ __device__ __forceinline__ int tiled_swz(int r) {
 // NT: weights loaded with the streaming cache policy (decode tiles, where each weight byte is
 // read by one block only). BFW: bf16 weights (the lm_head kept in bf16) in the 2 KB-per-step
 // tile layout, whose two 1 KB halves are the lo / hi operands an int8 tile dequantizes to: the
-// tiles are read from LDS as they are, with no scales, y = bf16(sum).
+// tiles are read from LDS as they are, with no scales, y = bf16(sum). ROWS: token rows of a block,
+// fewer than the BM its loads and LDS are laid out for: the same schedule with fewer MFMAs and
+// fragment reads, for token counts that would leave most of a block row of BM empty (tiled_shape).
 template <bool I8, int BM, int BN, int WGM, int WGN, int NST, bool GLU, bool NT = false,
-          bool BFW = false, bool STAGE_Y = false>
+          bool BFW = false, bool STAGE_Y = false, int ROWS = BM>
 __global__ void __launch_bounds__(64 * WGM * WGN)
 tiled_gemm_kernel(TiledArgs a) {
   using Acc = std::conditional_t<I8, i32x4, f32x4>;
@@ -104,8 +106,10 @@ tiled_gemm_kernel(TiledArgs a) {
   static_assert(!STAGE_Y || (!GLU && !BFW && (!I8 || (BM == 256 && BN == 256 && WGM == 2))),
                 "staged output: plain W8A16, or the W8A8 256 x 256 tile");
   constexpr int W = WGM * WGN;
-  constexpr int WM = BM / WGM, WN = BN / WGN;
+  constexpr int WM = ROWS / WGM, WN = BN / WGN;
   constexpr int TM = WM / 16, TN = WN / 16;
+  static_assert(ROWS <= BM && ROWS % (16 * WGM) == 0 && (ROWS == BM || !STAGE_Y),
+                "whole token tiles per wave");
   constexpr int ESZ = I8 ? 1 : 2;
   constexpr int XROW = 64 * ESZ;            // bytes of one x row per stage
   constexpr int XCH = XROW / 16;            // 16-byte chunks per row
@@ -174,7 +178,7 @@ tiled_gemm_kernel(TiledArgs a) {
   const int gm = min(a.mblocks - first_bm, kGroupM);
   const int tg = t - group * kGroupM * a.nblocks;
   const int bm = first_bm + tg % gm, bn = tg / gm;
-  const int m0 = bm * BM, n0 = bn * BN, rb0 = n0 / 16;
+  const int m0 = bm * ROWS, n0 = bn * BN, rb0 = n0 / 16;
 
   // The scales the block's epilogue applies, staged in LDS by direct-to-LDS loads issued before
   // the stage prologue (every later wait covers them): per-channel scales of its BN output rows
@@ -209,7 +213,7 @@ tiled_gemm_kernel(TiledArgs a) {
     }
   }
   // Buffer resources based at the block's first row / row tile, so 32-bit offsets suffice.
-  const int rows = min(BM, a.M - m0);
+  const int rows = min(ROWS, a.M - m0);
   const u32x4 xres = make_rsrc4(static_cast<const char*>(a.x) + (int64_t)m0 * a.ldx * ESZ,
                                 (uint32_t)(((int64_t)(rows - 1) * a.ldx + a.K) * ESZ));
   const int rtiles = min(WTILES, a.nrb - rb0);
@@ -514,7 +518,7 @@ tiled_gemm_kernel(TiledArgs a) {
     // 1 x 8 layout (each output adds its K stages in order, lo then hi half), so bit-identical.
     // The dequantization is duplicated over the two rows but runs beside MFMAs of the same wave;
     // the x fragment reads per stage halve (160 against 272 KB of LDS reads per block).
-    static_assert(NST == 3 && TN == 4 && TM == 8, "W8A16 256 x 256 ping-pong");
+    static_assert(NST == 3 && TN == 4 && TM <= 8, "W8A16 256 x 256 ping-pong");
     const bool row1 = wm == 1;
 #pragma unroll
     for (int i = 0; i < NST - 1; ++i) {
@@ -748,7 +752,7 @@ struct TiledShape {
   int bm, bn;
 };
 
-template <bool I8, int BM, int BN, bool GLU>
+template <bool I8, int BM, int BN, bool GLU, int ROWS = BM>
 static const void* tiled_fn() {
   // LDS per block: NST x (x stage + weight stage) <= 160 KB; 128 x 128 tiles keep two blocks
   // per CU. Wave layout 2 x 4, except the W8A16 128 x 256 tile: there 1 x 8 (128 x 32 per wave)
@@ -764,7 +768,7 @@ static const void* tiled_fn() {
   constexpr int wgm = (!I8 && BN == 256 && BM != 256) ? 1 : 2;
   static_assert(64 * wgm * (8 / wgm) == kTiledThreads, "8 waves");
   return reinterpret_cast<const void*>(
-      &tiled_gemm_kernel<I8, BM, BN, wgm, 8 / wgm, nst, GLU>);
+      &tiled_gemm_kernel<I8, BM, BN, wgm, 8 / wgm, nst, GLU, false, false, false, ROWS>);
 }
 
 // `decode`: a decode route's tile (one block row, M <= 64), whose weights stream with the nt
@@ -834,6 +838,12 @@ static const void* tiled_kernel_for(const TiledShape& sh, bool decode = false,
     }
     return tiled_fn<I8, 256, 256, GLU>();
   }
+  if (sh.bm == 224 && sh.bn == 256) return tiled_fn<I8, 256, 256, GLU, 224>();
+  if (sh.bm == 192 && sh.bn == 256) return tiled_fn<I8, 256, 256, GLU, 192>();
+  if (sh.bm == 112 && sh.bn == 256) {
+    if constexpr (I8) return nullptr;  // W8A16 only: one row of waves
+    else return tiled_fn<false, 128, 256, GLU, 112>();
+  }
   if (sh.bm == 256 && sh.bn == 192) {
     if constexpr (I8 || GLU) return nullptr;  // W8A16 without gate/up only (tiled_shape)
     else return tiled_fn<false, 256, 192, false>();
@@ -863,16 +873,28 @@ static const void* tiled_kernel_for(const TiledShape& sh, bool decode = false,
 // a quarter less padding than 128 x 128: on MI355X over gate_up (K 4096, N 28672) at 65 / 80 / 96
 // tokens 36-37 / 33.5 / 33.8 us against 38.3 / 38.5 / 39.5 us, fused gate_up 31.5-32.6 against
 // 37.6-38.8 us. Measured only there, so only launches of one such block row consider it.
-constexpr int kTileCands = 7;
+// The 224-, 192- and 112-row tiles (256 x 256 and 128 x 256 schedules over fewer token rows, ROWS) are
+// for token counts just past a multiple of a block row, where most of the last one would be
+// padding: their MFMAs shrink with the rows, their loads, barriers and dequantization do not, hence
+// the lower efficiencies, fitted so that none is picked where it measured slower. On MI355X, fused
+// gate/up (K 3072, N 16384) at 600 / 700 tokens 72.9 -> 63.2 / 75.6 -> 62 us in W8A16 and 39.7 ->
+// 35.8 / 40.4 -> 37.2 in W8A8; (K 4096, N 28672) at 300 / 1700 tokens 98 -> 86 / 406 -> 340 us; q/k/v
+// (N 6144) in W8A8 at 1500 / 3000 tokens 46.7 -> 41.5 / 93.8 -> 82.4; down_proj (K 14336) in W8A16 at
+// 3000 tokens 334 -> 288. The 112-row tile gains 3-5 % in W8A16 gate/up (417 tokens of K 3072: 44.6
+// -> 43.0) and lost 3-6 % on plain down_proj, so only gate/up considers it.
+constexpr int kTileCands = 10;
 constexpr TiledShape kTileCand[kTileCands] = {{256, 256}, {256, 128}, {128, 256}, {128, 128},
-                                              {64, 128},  {256, 192}, {96, 128}};
-constexpr double kTileEff16[kTileCands] = {1.0, 0.86, 0.87, 0.835, 0.6, 0.92, 0.75};
+                                              {64, 128},  {256, 192}, {96, 128},  {224, 256},
+                                              {192, 256}, {112, 256}};
+constexpr double kTileEff16[kTileCands] = {1.0,  0.86, 0.87, 0.835, 0.6,
+                                           0.92, 0.75, 0.92, 0.87,  0.84};
 // (256 x 192 and 96 x 128 serve W8A16 only.)
 // W8A8 re-measured once its 256 x 256 tile ran ping-pong with LDS-staged scales (averages over
 // the four shapes at M = 8192: 256 x 128 0.76, 128 x 256 0.80, 128 x 128 0.72); the picks that
 // changed (gate_up at M = 384, q/k/v at 2048, o_proj and down_proj at 3072: 256 x 256 instead of
 // 128 x 128) measured 11-19 % faster.
-constexpr double kTileEff8[kTileCands] = {1.0, 0.76, 0.80, 0.72, 0.6, 0.926, 0.75};
+constexpr double kTileEff8[kTileCands] = {1.0,   0.76, 0.80, 0.72, 0.6,
+                                          0.926, 0.75, 0.92, 0.87, 0.80};
 
 // One round of candidate i on every CU, in the cost model's units.
 template <bool I8>
@@ -890,6 +912,7 @@ static TiledShape tiled_shape(int64_t M, int64_t N, int cus, double* cost_out = 
     // launches at 4096), and never for gate/up (2 x 4 waves of 3 row tiles: not pairs).
     if (kTileCand[i].bn == 192 && (I8 || glu)) continue;
     if (kTileCand[i].bm == 96 && (I8 || M > 96)) continue;  // W8A16, one block row only
+    if (kTileCand[i].bm == 112 && (I8 || !glu)) continue;  // W8A16 gate/up only
     const int64_t blocks = ceil_div(M, kTileCand[i].bm) * ceil_div(N, kTileCand[i].bn);
     const double cost = (double)ceil_div(blocks, (int64_t)cus) * tile_round_cost<I8>(i);
     if (cost < best_cost * 0.999) {

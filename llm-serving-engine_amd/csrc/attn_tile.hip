@@ -34,11 +34,15 @@
 // Order of summation: tiles 2 j + s of stream s in order, then the two streams. It depends on the
 // row's own entry only.
 //
-// Measured on MI355X: three fresh prompts of 1285-1321 tokens, 32 heads over 8, 268 -> 66 us (640
+// Measured on MI355X: three fresh prompts of 1285-1321 tokens, 32 heads over 8, 268 -> 71 us (590
 // TFLOP/s of the causal half; a dense bf16 product of 8192^3 reaches 1434); a 735-token chunk behind
-// 1291 positions beside 40 decode rows, 24 heads over 8, 170 -> 98 us, of which this kernel about 40.
-// A phase takes 1300-1600 clocks of which 1024 are MFMA issue; an item's first loads and its
-// merge another 10000 or so, about a third of the time at these prompt lengths.
+// 1291 positions beside 40 decode rows, 24 heads over 8, 170 -> 91 us, of which this kernel 38 (and
+// attention.hip's, with its entries in order of length, 53). A phase takes 1300-1600 clocks of which
+// 1024 are MFMA issue; an item's first loads and its merge another 10000 or so, about a third of
+// the time at these prompt lengths. Without gain, against 66-68 us: the next item's first loads
+// issued before the merge (69 us); the tiles of consecutive items in one pipeline (73-105 us: the
+// softmax phase grows by the item cursors and the waits for Q); the loads in pairs between the
+// exponentials (68.5 us).
 #include <algorithm>
 #include <type_traits>
 
@@ -53,10 +57,19 @@ constexpr int kTileBytesKV = kTileKeys * 256;
 constexpr int kTileMaxEntries = 1024;  // entries of one launch (their tile counts lie in LDS)
 constexpr int kTileMaxLevels = 1024;
 constexpr int kTileListMax = 512;  // items of a workgroup whose list lies in LDS at a time
-// A row's reference m (probabilities are exp2(s - m)) moves to a larger score only when that is
-// more than this above it: probabilities then stay below 2^8, which costs no precision in bf16 or
-// fp32, and O is rescaled a few times per item instead of at nearly every tile.
-constexpr float kRescale = 8.0f;
+// A row's reference m (probabilities are exp2(s - m)) is its running maximum plus what makes it a whole
+// number above the tile's own maximum, so that the tile's largest probability is a power of two and
+// is rounded to bf16 without error; tiles whose maximum lies more than kAlign below it keep m. Relative
+// error against fp64 before the output is rounded (a model of the arithmetic, 1300 keys; scores of
+// standard deviation 1 and, where few keys matter, 3): 0.00125 and 0.00028; with the running
+// maximum itself 0.00142 and 0.00049 (the key-streaming kernel, which has one in each of 8 parts: 0.00131
+// and 0.00034); with one that lags by up to 8, which saves most rescales of O and 3 us of 70,
+// 0.00161 and 0.00142.
+constexpr float kAlign = 9.0f;
+// The exponent s - m is one fused multiply-add of the unscaled score, while m holds a rounded product:
+// the largest score's exponent is off by that rounding, at most 2^-10 up to this magnitude of m (no
+// bf16 probability changes). Past it the product is rounded first, as m's was.
+constexpr float kFarScore = 16384.0f;
 
 struct AttnTileArgs {
   int e0, entries;  // this launch's entries e0 .. e0 + entries - 1
@@ -311,7 +324,7 @@ attn_tile_kernel(PagedAttnArgs a, AttnTileArgs t) {
 
     const float sc = a.scale_log2 == 0.0f ? 1.0f : __builtin_fabsf(a.scale_log2);
     bf16x8 qf[8];
-    float m_run = NEG_INF, l_run = 0.0f;
+    float m_run = NEG_INF, m_max = NEG_INF, l_run = 0.0f;
     f32x16 oacc[4], st[2];
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -373,6 +386,7 @@ attn_tile_kernel(PagedAttnArgs a, AttnTileArgs t) {
     const std::false_type off{};
     // The softmax of st, tile j's scores: probabilities to pa, the running state and O rescaled.
     auto softmax = [&](int j) {
+#pragma clang fp contract(off)  // the maximum is a rounded product wherever it is used
       const int n0 = kTileKeys * (2 * j + stream);
       if (n0 + kTileKeys - 1 > all_see) {
         const int rel = lim - n0 - 4 * half;
@@ -389,24 +403,30 @@ attn_tile_kernel(PagedAttnArgs a, AttnTileArgs t) {
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[b][i]);
       const Halves hm = both_halves(mx);
       const float m_tile = fmaxf(hm.a, hm.b) * sc;
-      const float m_new = m_tile > m_run + kRescale ? m_tile : m_run;
+      m_max = fmaxf(m_max, m_tile);
+      const float below = m_max - m_tile;  // not <= kAlign where no key is seen yet (NaN)
+      const float m_new = below <= kAlign ? m_tile + __builtin_ceilf(below) : m_run;
       const float mref = m_new == NEG_INF ? 0.0f : m_new;  // a row with no key yet keeps p = 0
       const float alpha = m_new == m_run ? 1.0f : exp2_fast(m_run - mref);
+      float mul = sc, sub = mref;
+      if (__ballot(__builtin_fabsf(mref) > kFarScore)) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) st[b][i] = st[b][i] * sc - mref;
+        mul = 1.0f, sub = 0.0f;
+      }
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          st[b][i] = exp2_fast(__builtin_fmaf(st[b][i], sc, -mref));
-        }
+        for (int i = 0; i < 16; ++i) st[b][i] = exp2_fast(__builtin_fmaf(st[b][i], mul, -sub));
       l_run *= alpha;
       m_run = m_new;
       to_pa(0);
-      if (__ballot(alpha != 1.0f)) {
 #pragma unroll
-        for (int d = 0; d < 4; ++d)
+      for (int d = 0; d < 4; ++d)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
-      }
+        for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
     };
 
     if (steps > 0) {

@@ -8,6 +8,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from oracle import numerics as ora
 from test_gpu_attention import _case, _check, _run
 
 pytestmark = pytest.mark.gpu
@@ -45,6 +46,32 @@ def test_block_sizes(pkg, dev, block_size):
     entries = [(150, 77, 227), (1, 300, 301), (64, 0, 64), (5, 100, 105)]
     _check(pkg, dev, _case(300 + block_size, entries, h=8, h_kv=2, block_size=block_size),
            f"block {block_size}")
+
+
+@pytest.mark.parametrize("log2_q", [2, 12, 40, -40])
+def test_peaked_and_flat_scores(pkg, dev, log2_q):
+    """Scores of which few keys, one key (from 2^12 on rounding the scaled maximum moves it by more than
+    a probability's rounding, at 2^40 by more than fp32's range of exponents) and every key
+    alike matter."""
+    c = _case(450, [(150, 450, 600), (64, 0, 64)], h=8, h_kv=2)
+    c["q"] = ora.f32_to_bf16_bits(ora.bf16_bits_to_f32(c["q"]) * np.float32(2.0 ** log2_q))
+    _check(pkg, dev, c, f"q x 2^{log2_q}")
+
+
+def test_the_largest_probabilities_are_exact(pkg, dev):
+    """Few keys matter: each tile's largest probability is rounded to bf16 without error, so the
+    relative error stays near that of the output's own rounding (0.00165). Over 1300 keys the other
+    probabilities add 0.0003; with a reference that is not a whole number from the maximum they
+    would all add 0.0014. The bound allows them 0.0007."""
+    c = _case(460, [(100, 1200, 1300)], h=8, h_kv=2)
+    c["q"] = ora.f32_to_bf16_bits(ora.bf16_bits_to_f32(c["q"]) * np.float32(3))
+    o = ora.bf16_bits_to_f32(_run(pkg, dev, c)).astype(np.float64)
+    golden, _ = ora.paged_attention_golden(c["q"], c["kp"], c["vp"], c["table"], c["ctx"], c["qo"],
+                                           c["qs"], c["ql"], c["bs"])
+    golden = np.asarray(golden, np.float64)
+    rounded = ora.bf16_bits_to_f32(ora.f32_to_bf16_bits(golden.astype(np.float32)))
+    rms = lambda a: float(np.sqrt((a ** 2).mean() / (golden ** 2).mean()))  # noqa: E731
+    assert rms(o - golden) <= np.hypot(rms(rounded - golden), 0.0007)
 
 
 def test_rows_that_see_no_key(pkg, dev):

@@ -219,7 +219,8 @@ class DecodeRunner:
         pool = None
         if self.k_pool is not None:
             pool = (self.k_pool[i], self.v_pool[i], self.tables[rows])
-        if self._fused and nseq * ntok <= 65535:
+        # Only a slice of the cache is a view that the kernel can write through.
+        if self._fused and isinstance(rows, slice) and nseq * ntok <= 65535:
             q = ops.rope_kv(q[0], k[0], v[0], *rope, self.n_heads, self.n_kv, nseq, start,
                             (self.k_cache[i][rows], self.v_cache[i][rows]), pool)
         else:

@@ -132,3 +132,23 @@ def test_whole_step_replays_from_a_graph(runner, dev):
             assert torch.equal(again, eager), f"eager after replay {i}"
     finally:
         runner.use_attention("torch")
+
+
+@pytest.mark.parametrize("rows", [[4, 5, 6], torch.tensor([4, 5, 6])])
+def test_indexed_rows_write_their_cache(runner, dev, rows):
+    """Sequences given by index, whose cache rows are a copy and not a view: the same K/V writes and
+    the same hidden states as the slice of them."""
+    if runner.int8 is None:
+        runner.quantize("int8")
+    runner.use("int8")
+    runner.use_attention("torch")
+    gen = torch.Generator().manual_seed(17)
+    tok = torch.randint(0, runner.model.config.vocab_size, (3, 1), generator=gen).to(dev)
+    want = runner.forward(tok, 36, slice(4, 7))
+    caches = [(c, c[4:7, :, 36].clone()) for c in (*runner.k_cache, *runner.v_cache)]
+    for c, _ in caches:
+        c[4:7, :, 36] = 0
+    got = runner.forward(tok, 36, rows)
+    assert torch.equal(got, want)
+    for c, kv in caches:
+        assert torch.equal(c[4:7, :, 36], kv)

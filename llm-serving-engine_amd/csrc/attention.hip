@@ -112,6 +112,79 @@ __device__ __forceinline__ int attn_sorted_entry(const PagedAttnArgs& a, int slo
   return __ffsll(__ballot(rank == slot && lane < a.entries)) - 1;
 }
 
+// Sum over the lanes up to and including each.
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15, 31
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
+// Item p of the compact order: first every tile of the entries that have several, then one slot per
+// entry for those of a single tile (kAttnCompact: at most 64 entries, none of them long). False:
+// no such item.
+__device__ __forceinline__ bool attn_compact_item(const PagedAttnArgs& a, int p, int& e, int& qt) {
+  const int lane = threadIdx.x & 63;
+  const int qlen = lane < a.entries ? a.q_len[lane] : 0;
+  const int tiles = qlen > a.tq ? min((qlen + a.tq - 1) / a.tq, a.qtiles) : 0;
+  const int scan = wave_scan(tiles);
+  const int total = __builtin_amdgcn_readlane(scan, 63);
+  if (p < total) {
+    const int before = scan - tiles;
+    e = __ffsll(__ballot((unsigned)(p - before) < (unsigned)tiles)) - 1;
+    qt = p - __builtin_amdgcn_readlane(before, e);
+    return true;
+  }
+  p -= total;
+  if (p >= a.entries) return false;
+  e = a.sorted ? attn_sorted_entry(a, p) : p;
+  qt = 0;
+  return __builtin_amdgcn_readlane(qlen, e) <= a.tq;
+}
+
+// Item b of an entry's HKV x tiles x chunks in a split launch (see attn_order).
+__device__ __forceinline__ void attn_split_item(const PagedAttnArgs& a, int b, int tiles, int chunks,
+                                                int& kvh, int& qt, int& part) {
+  if (a.HKV % 8 == 0) {
+    kvh = b % a.HKV;
+    b /= a.HKV;
+    qt = b % tiles;
+    part = b / tiles;
+  } else {
+    part = b % chunks;
+    b /= chunks;
+    qt = b % tiles;
+    kvh = b / tiles;
+  }
+}
+
+// Item b of a split launch without gaps, entry by entry (kAttnCompactSplit: at most 64 entries).
+// False: no such item.
+__device__ __forceinline__ bool attn_compact_split_item(const PagedAttnArgs& a, int b, int& kvh,
+                                                        int& e, int& qt, int& part) {
+  const int lane = threadIdx.x & 63;
+  int tiles = 0, chunks = 0;
+  if (lane < a.entries) {
+    const int qlen = a.q_len[lane], ctx = a.context_len[lane];
+    if (qlen > 0 && !(a.tiled && attn_is_long((int64_t)qlen * a.G, ctx))) {
+      tiles = min((qlen + a.tq - 1) / a.tq, a.qtiles);
+      chunks = min(attn_chunks(min(a.query_offset[lane] + qlen, ctx)), a.parts);
+    }
+  }
+  const int items = a.HKV * tiles * chunks, before = wave_scan(items) - items;
+  const unsigned long long mine = __ballot((unsigned)(b - before) < (unsigned)items);
+  if (!mine) return false;
+  e = __ffsll(mine) - 1;
+  b -= __builtin_amdgcn_readlane(before, e);
+  chunks = __builtin_amdgcn_readlane(chunks, e);
+  tiles = __builtin_amdgcn_readlane(tiles, e);
+  attn_split_item(a, b, tiles, chunks, kvh, qt, part);
+  return true;
+}
+
 // NT: K and V stream with the nt cache policy; used when each K/V row is read by one workgroup
 // only (one query tile: decode). POW2: block_size is a power of two (a shift finds a key's block).
 template <int D, bool NT, bool POW2>
@@ -134,18 +207,33 @@ paged_attn_kernel(PagedAttnArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, grp = lane >> 4;
 
-  // K/V heads run fastest and query tiles slowest: consecutive workgroups go to the 8 XCDs in turn,
-  // and of a mixed batch only the first tile of most entries (and, split, the first chunks) exists.
-  // With tiles or chunks fastest, 16 tiles put all decode rows on one XCD.
-  int b = blockIdx.x;
-  const int kvh = b % a.HKV;
-  b /= a.HKV;
-  int e = b % a.entries;
-  b /= a.entries;
-  const int part = b % a.parts;
-  const int qt = b / a.parts;
+  // This workgroup's item; the order of the grid is the host's choice (attn_order).
+  int b = blockIdx.x, kvh, e, qt = 0, part = 0;
+  if (a.order == kAttnCompact) {
+    kvh = b % a.HKV;
+    if (!attn_compact_item(a, b / a.HKV, e, qt)) return;
+  } else if (a.order == kAttnCompactSplit) {
+    if (!attn_compact_split_item(a, b, kvh, e, qt, part)) return;
+  } else if (a.order == kAttnByTile) {
+    const int items = a.HKV * a.qtiles * a.parts;
+    e = b / items;
+    attn_split_item(a, b - e * items, a.qtiles, a.parts, kvh, qt, part);
+  } else {
+    const int first = a.entries * a.HKV;
+    const bool later = a.order == kAttnFirstTiles && b >= first;
+    if (later) b -= first;
+    kvh = b % a.HKV;
+    b /= a.HKV;
+    if (later) {
+      qt = 1 + b % (a.qtiles - 1);
+      e = b / (a.qtiles - 1);
+    } else {
+      e = b % a.entries;
+      part = b / a.entries;
+      if (a.sorted) e = attn_sorted_entry(a, e);
+    }
+  }
   const int G = a.G, TQ = a.tq;
-  if (a.sorted && qt == 0) e = attn_sorted_entry(a, e);
   const int qlen = a.q_len[e];
   if (qt * TQ >= qlen) return;
   const int ctx = a.context_len[e];
@@ -396,11 +484,37 @@ paged_attn_merge(PagedAttnArgs a) {
 // ---- host side -----------------------------------------------------------------------------
 
 struct AttnPlan {
-  int tq, qtiles, parts;
+  int tq, qtiles, parts, order;
   bool tiled;       // some entry may be the row-tiled kernel's
   int64_t short_q;  // the most query rows of an entry that is not
   int64_t ws_o_bytes, ws_bytes;
 };
+
+// The order of the grid. Consecutive workgroups go to the 8 XCDs in turn and, inside an XCD, to its
+// 32 CUs in turn, so where only some (entry, tile, chunk) slots hold work, their spacing decides how
+// evenly it spreads. With several query tiles per entry (a short prompt chunk), measured on MI355X against
+// one order for every launch (K/V heads fastest, then entries, chunks, tiles), and with chunks, then
+// tiles fastest, us; HKV = 8:
+//  * Split over chunks (attn_split_item): heads, then tiles, then chunks, so that the tiles that read a
+//    chunk are in flight together and on one XCD, whose L2 holds its K and V: 60 tokens behind 32000
+//    positions, 24 query heads, 148 (219 and 149); 8 chunks of 32 tokens behind 1000, 39 (35 and 53). With
+//    fewer heads than XCDs, chunks fastest puts a chunk on one XCD. From two entries on without the
+//    slots that hold no work: a 16-token chunk beside 12 decode rows 23 (24 and 54).
+//  * Unsplit: the first tiles (all that decode rows have) as in decode, then the others entry by entry. With
+//    tiles slowest a chunk among 63 decode rows has its tiles 512 slots apart, on one CU of each XCD;
+//    with tiles fastest 16 or 32 tiles put every decode row on one XCD (a 16-token chunk beside 63
+//    decode rows 64 (60 and 163)).
+//  * There, with 17 to 64 entries of which none is row-tiled: the items of entries of several tiles first,
+//    without gaps. They run longest, and after the decode rows they would start last: a 40-token
+//    chunk behind 2000 positions beside 63 decode rows 38 (65 and 41), 60 tokens behind 8000, 124
+//    (187 and 138). Finding an item takes 0.5 us or less, which fewer entries, whose workgroups all
+//    start at once, would not win back.
+static int attn_order(int64_t entries, int64_t HKV, const AttnPlan& pl) {
+  if (pl.qtiles == 1) return kAttnByEntry;
+  if (pl.parts > 1) return entries > 1 && entries <= 64 ? kAttnCompactSplit : kAttnByTile;
+  const bool fits = entries * HKV * (pl.qtiles + 1) <= 0x7fffffff;  // one slot more per entry
+  return !pl.tiled && fits && entries > 16 && entries <= 64 ? kAttnCompact : kAttnFirstTiles;
+}
 
 // One workgroup per (entry, K/V head, query tile) item once those fill the CUs twice over;
 // otherwise, when the table's context bound (max_blocks x block_size) spans 2..kAttnMaxSplit
@@ -419,6 +533,7 @@ static AttnPlan attn_plan(int64_t entries, int64_t H, int64_t HKV, int64_t D, in
   pl.parts = items > 0 && items < 2 * (int64_t)cus && chunks > 1 && chunks <= kAttnMaxSplit
                  ? (int)chunks
                  : 1;
+  pl.order = attn_order(entries, HKV, pl);
   if (pl.parts > 1) {
     const int64_t slots = (int64_t)pl.parts * entries * H * pl.short_q;
     pl.ws_o_bytes = slots * D * 4;
@@ -486,7 +601,9 @@ int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const 
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   a.ws_o = pl.parts > 1 ? static_cast<float*>(ws) : nullptr;
   a.ws_ml = pl.parts > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + pl.ws_o_bytes) : nullptr;
-  const int64_t blocks = (int64_t)a.entries * a.HKV * pl.qtiles * pl.parts;
+  a.order = pl.order;
+  const int64_t blocks =
+      (int64_t)a.entries * a.HKV * (pl.qtiles + (pl.order == kAttnCompact)) * pl.parts;
   if (blocks > 0x7fffffff ||
       (int64_t)a.entries * a.HKV * ceil_div(max_q_len, pl.tq) > 0x7fffffff)
     return LSE_E_RANGE;

@@ -614,9 +614,11 @@ int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const 
   }
   // Measured on MI355X: 64 decode rows over 8 K/V heads, contexts 256 to 2048 (300 MB of K and V),
   // 74.6 us in the given order, 58.9 sorted; 40 rows beside a 735-token chunk 98 and 88; 64 rows of one
-  // context the same within 0.2 us. Split launches (few items) start everything at once anyway.
+  // context the same within 0.7 us, which is what ranking costs: 2 to 32 rows of up to 256 positions 6.0
+  // to 11.6 us and 6.7 to 12.2. So only where some CU gets several items and contexts may be long; split
+  // launches (few items) start everything at once anyway.
   const int64_t cus = attn_cus(), items = (int64_t)a.entries * a.HKV;
-  a.sorted = a.parts == 1 && a.entries > 1 && a.entries <= 64;
+  a.sorted = a.parts == 1 && a.entries <= 64 && items > cus && max_ctx > 256;
   a.first_round = items > cus && items <= 2 * cus && cus % a.HKV == 0 ? (int)(cus / a.HKV) : 0;
   void* args[] = {&a};
   const bool pow2 = a.bs_shift >= 0;

@@ -549,6 +549,15 @@ attn_tile_kernel(PagedAttnArgs a, AttnTileArgs t) {
   }
 }
 
+// One workgroup per CU, or per item where those are fewer, in whole rounds over the 8 XCDs: rounded up
+// (workgroups without an item leave at once), since rounding down gave some workgroups two items
+// one after the other while most CUs had none (200 tokens behind 2000 positions, 8 heads over 2: 14
+// items, 41 us in 16 workgroups, 73 in 8).
+static int64_t attn_tile_grid(int64_t items, int cus) {
+  const int64_t grid = std::min<int64_t>(cus, ceil_div(items, 8) * 8);
+  return grid >= 8 ? grid & ~(int64_t)7 : grid;
+}
+
 int launch_attn_tile(const PagedAttnArgs& a0, int cus, hipStream_t stream) {
   PagedAttnArgs a = a0;
   const int64_t tiles = ceil_div((int64_t)a.max_q_len * a.G, kTileRowsQ);
@@ -560,8 +569,7 @@ int launch_attn_tile(const PagedAttnArgs& a0, int cus, hipStream_t stream) {
                                    : reinterpret_cast<const void*>(&attn_tile_kernel<false>);
   for (t.e0 = 0; t.e0 < a.entries; t.e0 += kTileMaxEntries) {
     t.entries = std::min(kTileMaxEntries, a.entries - t.e0);
-    int64_t grid = std::min<int64_t>(cus, t.entries * tiles * a.HKV);
-    if (grid >= 8) grid &= ~(int64_t)7;
+    const int64_t grid = attn_tile_grid(t.entries * tiles * a.HKV, cus);
     void* args[] = {&a, &t};
     const hipError_t err = hipLaunchKernel(fn, dim3((unsigned)grid), dim3(64 * kTileWaves), args, 0,
                                            stream);

@@ -28,7 +28,6 @@ struct PagedAttnArgs {
   int bs_shift;      // log2(block_size) when it is a power of two, else -1
   int tq;            // query tokens per tile: floor(16 / G)
   int qtiles;        // ceil(max_q_len / tq)
-  int order;         // of the grid
   int parts;         // 1: a workgroup folds every chunk of its item; > 1: one chunk per workgroup
   int sorted;        // entries are taken in descending order of context length...
   int first_round;   // ...and, where > 0, those from this rank on in ascending order

@@ -185,12 +185,14 @@ __device__ __forceinline__ bool attn_compact_split_item(const PagedAttnArgs& a, 
   return true;
 }
 
-// NT: K and V stream with the nt cache policy; used when each K/V row is read by one workgroup
-// only (one query tile: decode). POW2: block_size is a power of two (a shift finds a key's block).
-template <int D, bool NT, bool POW2>
+// ORDER: of the grid (attn_order). NT: K and V stream with the nt cache policy, where each K/V row is read
+// by one workgroup only (one query tile: decode). POW2: block_size is a power of two (a shift finds a
+// key's block).
+template <int D, int ORDER, bool POW2>
 __global__ void __launch_bounds__(64 * kAttnWaves)
 paged_attn_kernel(PagedAttnArgs a) {
   static_assert(D == 128, "head_dim 128: 16 chunks of 16 bytes per K/V row");
+  constexpr bool NT = ORDER == kAttnByEntry;
   constexpr int W = kAttnWaves, KT = kAttnKeys, KK = D / 32, DT = D / 16;
   constexpr int VROWB = 2 * D;  // bytes of one V row in LDS
   constexpr float NEG_INF = -__builtin_huge_valf();
@@ -207,20 +209,20 @@ paged_attn_kernel(PagedAttnArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, grp = lane >> 4;
 
-  // This workgroup's item; the order of the grid is the host's choice (attn_order).
+  // This workgroup's item.
   int b = blockIdx.x, kvh, e, qt = 0, part = 0;
-  if (a.order == kAttnCompact) {
+  if constexpr (ORDER == kAttnCompact) {
     kvh = b % a.HKV;
     if (!attn_compact_item(a, b / a.HKV, e, qt)) return;
-  } else if (a.order == kAttnCompactSplit) {
+  } else if constexpr (ORDER == kAttnCompactSplit) {
     if (!attn_compact_split_item(a, b, kvh, e, qt, part)) return;
-  } else if (a.order == kAttnByTile) {
+  } else if constexpr (ORDER == kAttnByTile) {
     const int items = a.HKV * a.qtiles * a.parts;
     e = b / items;
     attn_split_item(a, b - e * items, a.qtiles, a.parts, kvh, qt, part);
   } else {
     const int first = a.entries * a.HKV;
-    const bool later = a.order == kAttnFirstTiles && b >= first;
+    const bool later = ORDER == kAttnFirstTiles && b >= first;
     if (later) b -= first;
     kvh = b % a.HKV;
     b /= a.HKV;
@@ -560,6 +562,19 @@ int64_t paged_attention_workspace_bytes(int64_t entries, int64_t H, int64_t HKV,
   return attn_plan(entries, H, HKV, D, max_q_len, max_ctx, attn_cus()).ws_bytes;
 }
 
+template <bool POW2>
+static const void* attn_kernel(int order) {
+  switch (order) {
+    case kAttnByEntry: return reinterpret_cast<const void*>(&paged_attn_kernel<128, kAttnByEntry, POW2>);
+    case kAttnByTile: return reinterpret_cast<const void*>(&paged_attn_kernel<128, kAttnByTile, POW2>);
+    case kAttnFirstTiles:
+      return reinterpret_cast<const void*>(&paged_attn_kernel<128, kAttnFirstTiles, POW2>);
+    case kAttnCompact: return reinterpret_cast<const void*>(&paged_attn_kernel<128, kAttnCompact, POW2>);
+    default:
+      return reinterpret_cast<const void*>(&paged_attn_kernel<128, kAttnCompactSplit, POW2>);
+  }
+}
+
 int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const uint16_t* k_pool,
                            const uint16_t* v_pool, int64_t sb, int64_t sw, int64_t sh,
                            const int32_t* block_table, int64_t sbt, const int32_t* context_len,
@@ -604,7 +619,6 @@ int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const 
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   a.ws_o = pl.parts > 1 ? static_cast<float*>(ws) : nullptr;
   a.ws_ml = pl.parts > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + pl.ws_o_bytes) : nullptr;
-  a.order = pl.order;
   const int64_t blocks =
       (int64_t)a.entries * a.HKV * (pl.qtiles + (pl.order == kAttnCompact)) * pl.parts;
   if (blocks > 0x7fffffff ||
@@ -624,13 +638,7 @@ int launch_paged_attention(const uint16_t* q, int64_t sq_h, int64_t sq_t, const 
   a.sorted = a.parts == 1 && a.entries <= 64 && items > cus && max_ctx > 256;
   a.first_round = items > cus && items <= 2 * cus && cus % a.HKV == 0 ? (int)(cus / a.HKV) : 0;
   void* args[] = {&a};
-  const bool pow2 = a.bs_shift >= 0;
-  const void* fn =
-      pl.qtiles == 1
-          ? (pow2 ? reinterpret_cast<const void*>(&paged_attn_kernel<128, true, true>)
-                  : reinterpret_cast<const void*>(&paged_attn_kernel<128, true, false>))
-          : (pow2 ? reinterpret_cast<const void*>(&paged_attn_kernel<128, false, true>)
-                  : reinterpret_cast<const void*>(&paged_attn_kernel<128, false, false>));
+  const void* fn = a.bs_shift >= 0 ? attn_kernel<true>(pl.order) : attn_kernel<false>(pl.order);
   hipError_t err = hipLaunchKernel(fn,
                                    dim3((unsigned)blocks), dim3(64 * kAttnWaves), args, 0, stream);
   if (err == hipSuccess && pl.parts > 1) {

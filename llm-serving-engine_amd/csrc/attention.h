@@ -37,17 +37,51 @@ struct PagedAttnArgs {
   int tiled;         // the row-tiled kernel runs too and takes the long entries (attn_is_long)
 };
 
-// Whether the row-tiled kernel takes an entry of `rows` = q_len x G query rows per K/V head; the
-// key-streaming kernel takes it otherwise. The choice depends on the entry alone, so a row's bits do
-// not depend on the rest of the call. Measured on MI355X (32 heads over 8; us, key-streaming against
-// row-tiled): 8 entries of 64 tokens behind 1000 positions 60.0 / 27.2, one of them 23.1 / 24.2; of
-// 32 tokens 49 / 26 and 22.5 / 24.3, fresh prompts of 32 tokens 6.7 / 11.5 (two launches), so 256 rows
-// is where it starts. A workgroup walks its rows' whole context, so a lone short chunk far into a
-// long one leaves the chip idle: one entry behind 8000 positions 55 / 98 at 64 tokens, 97 / 99 at 128,
-// 181 / 102 at 256.
-constexpr int kAttnTileRows = 256, kAttnTileRowsFar = 512, kAttnTileNear = 2048;
-__host__ __device__ inline bool attn_is_long(int64_t rows, int ctx) {
-  return rows >= kAttnTileRowsFar || (rows >= kAttnTileRows && ctx <= kAttnTileNear);
+// Whether the row-tiled kernel takes an entry of q_len tokens; the key-streaming kernel takes it
+// otherwise. The choice depends on the entry and the heads alone, so a row's bits do not depend on the
+// rest of the call, and it is fitted so that an entry alone in its call is not slower for it (among
+// others it gains more). The key-streaming kernel's time grows with the (query row, key) pairs; the
+// row-tiled one's, with fewer items than CUs, with the context its workgroups walk, 13 us per 1000
+// positions, on top of some 12 us for both launches. Measured on MI355X, us, key-streaming / row-tiled:
+//  * fresh prompts, 32 heads over 8: one of 64 tokens 6 / 12, 128: 7 / 12, 256: 12 / 14, 320: 19 / 16, 512:
+//    27 / 18; four of 128: 16 / 13, of 256: 36 / 16; one of 512, 8 heads over 2: 12 / 17; of 2048: 71 / 37;
+//  * one entry behind 500 positions, 32 over 8: 128 tokens 14 / 19, 256: 22 / 20;
+//  * behind 2000: 64 tokens 31 / 33, 128: 44 / 39; 8 heads over 2, 128: 22 / 39, 512: 49 / 45; 4 over 1,
+//    512: 30 / 43, 1024: 49 / 50;
+//  * behind 8000: 32 over 8, 128 tokens 101 / 114, 200: 163 / 116; 4 over 1, 512: 73 / 119, 2048: 207 / 136.
+// An item is 128 rows of a K/V head, so fewer than 256 would leave much of them idle. With fewer than 8
+// K/V heads (a shard's), the same work is more tokens, whose workgroups walk more of their own keys: there
+// the gain alone is small (8 over 2, 512 tokens behind 2000 positions, above), and beside decode rows,
+// which run after the row-tiled kernel and beside the other, it turns into a loss (50 / 72).
+constexpr int kAttnTileRows = 256;            // query rows per K/V head
+constexpr int kAttnTileHeads = 4096;          // q_len x H, from which with kAttnTilePairs...
+constexpr int kAttnTileHeadsFar = 5120;       // ...(contexts longer than kAttnTileNear)
+constexpr int kAttnTileHeadsFew = 8192;       // ...(fewer than 8 K/V heads)
+constexpr int kAttnTileNear = 4096;
+constexpr int64_t kAttnTilePairs = 4000000;   // (query row, key) pairs over all heads
+constexpr int kAttnTileAlways = 10240;        // q_len x H, from which in any case
+__host__ __device__ inline bool attn_is_long(int64_t q_len, int G, int HKV, int ctx) {
+  const int64_t rows = q_len * G, heads = rows * HKV;
+  const int from = HKV < 8 ? kAttnTileHeadsFew
+                           : ctx > kAttnTileNear ? kAttnTileHeadsFar : kAttnTileHeads;
+  return rows >= kAttnTileRows &&
+         (heads >= kAttnTileAlways ||
+          (heads >= from && heads * (2 * (int64_t)ctx - q_len) >= 2 * kAttnTilePairs));
+}
+// Whether a call may hold a long entry, from what the host knows: no more than max_q_len tokens, contexts
+// within the block table's max_ctx positions.
+inline bool attn_may_be_long(int64_t max_q_len, int G, int HKV, int64_t max_ctx) {
+  const int64_t rows = max_q_len * G, heads = rows * HKV;
+  const int64_t q = max_q_len < max_ctx ? max_q_len : max_ctx;
+  return rows >= kAttnTileRows &&
+         (heads >= kAttnTileAlways ||
+          (heads >= (HKV < 8 ? kAttnTileHeadsFew : kAttnTileHeads) &&
+           q * G * HKV * (2 * max_ctx - q) >= 2 * kAttnTilePairs));
+}
+// The most tokens of an entry that is not long whatever its context.
+inline int64_t attn_short_tokens(int G, int HKV) {
+  const int64_t by_heads = (kAttnTileAlways - 1) / (G * HKV), by_rows = (kAttnTileRows - 1) / G;
+  return by_heads > by_rows ? by_heads : by_rows;
 }
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));

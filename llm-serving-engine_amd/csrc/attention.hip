@@ -102,7 +102,7 @@ __device__ __forceinline__ int attn_sorted_entry(const PagedAttnArgs& a, int slo
   int key = -1;  // longer first, then the lower index
   if (lane < a.entries) {
     const int qlen = a.q_len[lane], ctx = a.context_len[lane];
-    const bool none = qlen == 0 || (a.tiled && attn_is_long((int64_t)qlen * a.G, ctx));
+    const bool none = qlen == 0 || (a.tiled && attn_is_long(qlen, a.G, a.HKV, ctx));
     key = ((none ? 0 : 1 + min(max(ctx, 0), (1 << 24) - 1)) << 6) + 63 - lane;
   }
   int rank = 0;
@@ -169,7 +169,7 @@ __device__ __forceinline__ bool attn_compact_split_item(const PagedAttnArgs& a, 
   int tiles = 0, chunks = 0;
   if (lane < a.entries) {
     const int qlen = a.q_len[lane], ctx = a.context_len[lane];
-    if (qlen > 0 && !(a.tiled && attn_is_long((int64_t)qlen * a.G, ctx))) {
+    if (qlen > 0 && !(a.tiled && attn_is_long(qlen, a.G, a.HKV, ctx))) {
       tiles = min((qlen + a.tq - 1) / a.tq, a.qtiles);
       chunks = min(attn_chunks(min(a.query_offset[lane] + qlen, ctx)), a.parts);
     }
@@ -239,7 +239,7 @@ paged_attn_kernel(PagedAttnArgs a) {
   const int qlen = a.q_len[e];
   if (qt * TQ >= qlen) return;
   const int ctx = a.context_len[e];
-  if (a.tiled && attn_is_long((int64_t)qlen * G, ctx)) return;
+  if (a.tiled && attn_is_long(qlen, G, a.HKV, ctx)) return;
   const int qo = a.query_offset[e], qs = a.q_start[e];
   const int end_n = attn_end(qo, qlen, ctx, qt, TQ);
   const int nch = attn_chunks(end_n);
@@ -469,7 +469,7 @@ paged_attn_merge(PagedAttnArgs a) {
   const int e = (int)(r / a.H);
   const int qlen = a.q_len[e];
   if (m >= qlen) return;
-  if (a.tiled && attn_is_long((int64_t)qlen * a.G, a.context_len[e])) return;
+  if (a.tiled && attn_is_long(qlen, a.G, a.HKV, a.context_len[e])) return;
   const int end_n = attn_end(a.query_offset[e], qlen, a.context_len[e], m / a.tq, a.tq);
   const int np = attn_chunks(end_n);
   const int64_t stride = (int64_t)a.entries * a.H * a.max_q_len;
@@ -488,7 +488,7 @@ paged_attn_merge(PagedAttnArgs a) {
 struct AttnPlan {
   int tq, qtiles, parts, order;
   bool tiled;       // some entry may be the row-tiled kernel's
-  int64_t short_q;  // the most query rows of an entry that is not
+  int64_t short_q;  // the most tokens of an entry that is not
   int64_t ws_o_bytes, ws_bytes;
 };
 
@@ -529,8 +529,8 @@ static AttnPlan attn_plan(int64_t entries, int64_t H, int64_t HKV, int64_t D, in
                           int64_t max_ctx, int cus) {
   AttnPlan pl{};
   const int64_t G = H / HKV;
-  pl.tiled = max_q_len * G >= kAttnTileRows;
-  pl.short_q = std::min<int64_t>(max_q_len, (kAttnTileRowsFar - 1) / G);
+  pl.tiled = attn_may_be_long(max_q_len, (int)G, (int)HKV, max_ctx);
+  pl.short_q = pl.tiled ? std::min<int64_t>(max_q_len, attn_short_tokens((int)G, (int)HKV)) : max_q_len;
   pl.tq = (int)(16 / (H / HKV));
   pl.qtiles = (int)ceil_div(pl.short_q, pl.tq);
   const int64_t items = entries * HKV * ceil_div(max_q_len, (int64_t)pl.tq);

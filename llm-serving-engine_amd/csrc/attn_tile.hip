@@ -174,8 +174,10 @@ attn_tile_kernel(PagedAttnArgs a, AttnTileArgs t) {
   // The work list: level l holds row tiles [l << sh, (l + 1) << sh) of every entry, and pre[l] is
   // the number of row tiles in the levels above it.
   for (int i = threadIdx.x; i < t.entries; i += 64 * kTileWaves) {
-    const int rows = a.q_len[t.e0 + i] * G;
-    ntile[i] = attn_is_long(rows, a.context_len[t.e0 + i]) ? (rows + kTileRowsQ - 1) / kTileRowsQ : 0;
+    const int qlen = a.q_len[t.e0 + i];
+    ntile[i] = attn_is_long(qlen, G, a.HKV, a.context_len[t.e0 + i])
+                   ? (qlen * G + kTileRowsQ - 1) / kTileRowsQ
+                   : 0;
   }
   __syncthreads();
   for (int l = threadIdx.x; l <= t.levels; l += 64 * kTileWaves) {

@@ -5,6 +5,9 @@ long ones. The tolerance is test_gpu_attention's (bf16 probabilities and output)
 
 from __future__ import annotations
 
+import re
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -13,39 +16,63 @@ from test_gpu_attention import _case, _check, _run
 
 pytestmark = pytest.mark.gpu
 
-FIRST_ROWS = 256  # query rows (tokens x heads of a K/V head) from which an entry is row-tiled...
-NEAR = 2048  # ...when its context is no longer than this; from twice the rows on in any case
+HEADER = Path(__file__).resolve().parent.parent / "llm-serving-engine_amd" / "csrc" / "attention.h"
+BOUND = {name: int(value) for name, value in
+         re.findall(r"constexpr \w+ kAttnTile(\w+) = (\d+);", HEADER.read_text())}
+WIDE = dict(h=160, h_kv=10)  # many heads, so that entries of 64 tokens are long
 
 
-@pytest.mark.parametrize("h,h_kv", [(4, 4), (6, 2), (8, 2), (10, 2), (16, 1)])
+def _long(c, e):
+    """Whether entry e of the case is the row-tiled kernel's, by the library's own bounds."""
+    n, ctx, h, h_kv = int(c["ql"][e]), int(c["ctx"][e]), c["q"].shape[0], c["kp"].shape[2]
+    start = "HeadsFew" if h_kv < 8 else "HeadsFar" if ctx > BOUND["Near"] else "Heads"
+    return n * (h // h_kv) >= BOUND["Rows"] and (
+        n * h >= BOUND["Always"]
+        or (n * h >= BOUND[start] and n * h * (2 * ctx - n) >= 2 * BOUND["Pairs"]))
+
+
+def _case_of(longs, *args, **kw):
+    """A case of which exactly the entries `longs` are the row-tiled kernel's."""
+    c = _case(*args, **kw)
+    assert [e for e in range(len(c["ql"])) if _long(c, e)] == longs
+    return c
+
+
+@pytest.mark.parametrize("h,h_kv", [(40, 40), (30, 10), (32, 8), (50, 10), (96, 8), (128, 8)])
 def test_first_length_and_tile_edges(pkg, dev, h, h_kv):
     """Entries on both sides of the first row-tiled length, and of the next row tile."""
     g = h // h_kv
-    first = -(-FIRST_ROWS // g)
-    lens = [first - 1, first, first + 1, (FIRST_ROWS + 128) // g, (FIRST_ROWS + 128) // g + 1]
+    first = max(-(-BOUND["Always"] // h), -(-BOUND["Rows"] // g))
+    tile = (first * g // 128 + 1) * 128
+    lens = [first - 1, first, first + 1, tile // g, tile // g + 1]
     entries = [(n, off, n + off) for n, off in zip(lens, [0, 0, 3, 64, 129])]
-    _check(pkg, dev, _case(100 + h, entries, h=h, h_kv=h_kv), f"H={h} H_KV={h_kv}")
+    c = _case_of([1, 2, 3, 4], 100 + h, entries, h=h, h_kv=h_kv)
+    _check(pkg, dev, c, f"H={h} H_KV={h_kv}")
 
 
 def test_far_chunks_start_later(pkg, dev):
-    """Entries on both sides of the context and row bounds, whose tiles span many key steps."""
-    entries = [(n, ctx - n, ctx) for n in (32, 63, 64) for ctx in (NEAR, NEAR + 1)]
-    _check(pkg, dev, _case(150, entries, h=8, h_kv=1), "far chunks")
+    """Entries on both sides of the bounds by context and by (row, key) pairs, whose tiles span many
+    key steps."""
+    entries = [(n, ctx - n, ctx) for n, ctx in [(128, 1040), (128, 1041), (127, 1100), (128, 4096),
+                                                (128, 4097), (159, 4097), (160, 4097)]]
+    _check(pkg, dev, _case_of([1, 3, 6], 150, entries, h=32, h_kv=8), "far chunks")
+    entries = [(n, 900, n + 900) for n in (127, 128)]
+    _check(pkg, dev, _case_of([1], 151, entries, h=64, h_kv=4), "few K/V heads")
 
 
 @pytest.mark.parametrize("end", [63, 64, 65, 127, 128, 129, 191, 192, 193, 257])
 def test_key_tile_edges(pkg, dev, end):
     """Contexts one short of and one over a key tile, a pair of tiles and the four in flight; the
     second entry's context ends before its own query rows do, so its rows see different ends."""
-    c = _case(200 + end, [(end, 0, end), (end, 11, end)], h=16, h_kv=2)
+    c = _case_of([0, 1], 200 + end, [(end, 0, end), (end, 11, end)], h=176, h_kv=11)
     _check(pkg, dev, c, f"end={end}")
 
 
 @pytest.mark.parametrize("block_size", [1, 7, 16, 24, 48, 64])
 def test_block_sizes(pkg, dev, block_size):
     entries = [(150, 77, 227), (1, 300, 301), (64, 0, 64), (5, 100, 105)]
-    _check(pkg, dev, _case(300 + block_size, entries, h=8, h_kv=2, block_size=block_size),
-           f"block {block_size}")
+    c = _case_of([0, 2], 300 + block_size, entries, **WIDE, block_size=block_size)
+    _check(pkg, dev, c, f"block {block_size}")
 
 
 @pytest.mark.parametrize("log2_q", [2, 12, 40, -40])
@@ -53,7 +80,7 @@ def test_peaked_and_flat_scores(pkg, dev, log2_q):
     """Scores of which few keys, one key (from 2^12 on rounding the scaled maximum moves it by more than
     a probability's rounding, at 2^40 by more than fp32's range of exponents) and every key
     alike matter."""
-    c = _case(450, [(150, 450, 600), (64, 0, 64)], h=8, h_kv=2)
+    c = _case_of([0, 1], 450, [(150, 450, 600), (64, 0, 64)], **WIDE)
     c["q"] = ora.f32_to_bf16_bits(ora.bf16_bits_to_f32(c["q"]) * np.float32(2.0 ** log2_q))
     _check(pkg, dev, c, f"q x 2^{log2_q}")
 
@@ -63,7 +90,7 @@ def test_the_largest_probabilities_are_exact(pkg, dev):
     relative error stays near that of the output's own rounding (0.00165). Over 1300 keys the other
     probabilities add 0.0003; with a reference that is not a whole number from the maximum they
     would all add 0.0014. The bound allows them 0.0007."""
-    c = _case(460, [(100, 1200, 1300)], h=8, h_kv=2)
+    c = _case_of([0], 460, [(100, 1200, 1300)], **WIDE)
     c["q"] = ora.f32_to_bf16_bits(ora.bf16_bits_to_f32(c["q"]) * np.float32(3))
     o = ora.bf16_bits_to_f32(_run(pkg, dev, c)).astype(np.float64)
     golden, _ = ora.paged_attention_golden(c["q"], c["kp"], c["vp"], c["table"], c["ctx"], c["qo"],
@@ -76,7 +103,7 @@ def test_the_largest_probabilities_are_exact(pkg, dev):
 
 def test_rows_that_see_no_key(pkg, dev):
     """An entry without any context gives zeros."""
-    c = _case(400, [(70, 0, 70), (80, 0, 80)], h=8, h_kv=2)
+    c = _case_of([0, 1], 400, [(70, 0, 70), (80, 0, 80)], **WIDE)
     c["ctx"] = np.array([70, 0], np.int32)
     o = _run(pkg, dev, c)
     assert not (o[:, 70:] & 0x7FFF).any()
@@ -87,7 +114,7 @@ def test_rows_do_not_depend_on_the_batch(pkg, dev):
     """A long entry's rows have the same bits alone, among decode rows and other prompts, with a
     larger max_q_len and a wider table; slots nobody owns hold NaN."""
     entries = [(1, 40, 41), (200, 100, 300), (90, 0, 90), (1, 700, 701), (65, 31, 96)]
-    c = _case(500, entries, h=8, h_kv=2, spare_blocks=5)
+    c = _case_of([1, 2, 4], 500, entries, **WIDE, spare_blocks=5)
     base = _check(pkg, dev, c, "batch")
     owned = np.zeros(c["kp"].shape[:2], bool)
     for e, ctx in enumerate(c["ctx"]):
@@ -107,18 +134,20 @@ def test_rows_do_not_depend_on_the_batch(pkg, dev):
 
 def test_more_entries_than_one_launch_holds(pkg, dev):
     """Over 1024 entries, a few of them long."""
-    entries = [(17 if e % 100 == 0 or e > 1026 else 1, 0, 17 if e % 100 == 0 or e > 1026 else 1)
-               for e in range(1030)]
-    _check(pkg, dev, _case(600, entries, h=16, h_kv=1), "1030 entries")
+    longs = [e for e in range(1030) if e % 200 == 0 or e > 1026]
+    entries = [(33, 0, 33) if e in longs else (1, 0, 1) for e in range(1030)]
+    _check(pkg, dev, _case_of(longs, 600, entries, h=320, h_kv=20), "1030 entries")
 
 
-@pytest.mark.parametrize("entries", [2, 33, 63, 64, 65])
+@pytest.mark.parametrize("entries", [2, 32, 33, 63, 64, 65])
 def test_entries_in_order_of_length(pkg, dev, entries):
     """Decode rows of different and equal contexts, with padding rows (q_len 0), on both sides of
-    the entry counts whose workgroups are ordered by length and paired on a CU."""
+    the entry counts whose workgroups are ordered by length and paired on a CU (from one more item
+    than CUs to 64 entries)."""
     rng = np.random.default_rng(entries)
-    ctx = rng.integers(1, 90, entries)
-    ctx[::3] = 40
+    ctx = rng.integers(1, 300, entries)
+    ctx[0] = 300  # a table of more than 256 positions
+    ctx[1::3] = 40
     c = _case(700 + entries, [(1, int(n) - 1, int(n)) for n in ctx], h=8, h_kv=8)
     base = _check(pkg, dev, c, f"{entries} entries")
     pad = dict(c, ql=c["ql"].copy(), ctx=c["ctx"].copy())

@@ -84,13 +84,15 @@ __device__ __forceinline__ f32x16 mfma32x32x16(bf16x8 a, bf16x8 b, f32x16 c) {
 
 // Four 16-byte global loads straight to LDS: lane l's bytes of load i land at lds + 1024 i + 16 l.
 // Not tracked by the compiler: ordered by explicit vmcnt waits and barriers. M0 (the LDS address) is
-// restored.
+// restored. A vector-memory read of an SGPR that a VALU instruction wrote (v_readlane of a spilled base,
+// v_readfirstlane) needs five wait states between the two, and the compiler does not look into the block:
+// its three instructions before the first load make five.
 __device__ __forceinline__ void dma4_saddr(uint32_t lds, const void* base, const uint32_t (&off)[4]) {
   uint32_t saved;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
+      "s_nop 2\n\t"
       "global_load_lds_dwordx4 %2, %6\n\t"
       "s_add_u32 m0, m0, 0x400\n\t"
       "s_nop 0\n\t"

@@ -99,12 +99,13 @@ constexpr int kNormThreads = 512;
 
 // One workgroup per row, thread t holding elements 8 t + 4096 i (i < NV): s = bf16(x + res) (or x),
 // y = bf16(w * bf16(s * r)), r = 1 / sqrt(mean(s^2) + eps), the roundings of LlamaRMSNorm
-// (modeling_llama.py:62-67). The sum of squares: each thread's in order, then a fixed tree.
+// (modeling_llama.py:62-67). The sum of squares: each thread's in order, then a fixed tree. `sum` may be x
+// or res: a thread reads all of its elements before it writes any.
 template <int NV>
 __global__ void __launch_bounds__(kNormThreads)
-add_rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ res,
-                   int64_t ldr, const uint16_t* __restrict__ w, float eps,
-                   uint16_t* __restrict__ sum, uint16_t* __restrict__ y, int K) {
+add_rmsnorm_kernel(const uint16_t* x, int64_t ldx, const uint16_t* res, int64_t ldr,
+                   const uint16_t* __restrict__ w, float eps, uint16_t* sum,
+                   uint16_t* __restrict__ y, int K) {
   __shared__ float red[kNormThreads / 64];
   const int64_t m = blockIdx.x;
   uint32_t u[NV][4], g[NV][4];
@@ -132,8 +133,14 @@ add_rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* 
       ss = __builtin_fmaf(lo, lo, ss);
       ss = __builtin_fmaf(hi, hi, ss);
     }
-    if (sum && k < K)
-      *reinterpret_cast<uint4*>(sum + m * K + k) = make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]);
+  }
+  if (sum) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int k = 8 * (threadIdx.x + kNormThreads * i);
+      if (k < K)
+        *reinterpret_cast<uint4*>(sum + m * K + k) = make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]);
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);

@@ -74,6 +74,23 @@ def test_add_rmsnorm(pkg, dev, m, k, residual):
     assert ulps.max() <= 2 and np.mean(ulps > 0) < 1e-3 + 1.0 / ulps.size
 
 
+@pytest.mark.parametrize("m,k", [(1, 8), (5, 4104), (3, 16384)])
+@pytest.mark.parametrize("into", ["x", "res"])
+def test_add_rmsnorm_in_place(pkg, dev, m, k, into):
+    """The sum written over one of its operands, as the C entry allows."""
+    gen = torch.Generator().manual_seed(m * k)
+    x, r = _bf16(gen, m, k).to(dev), _bf16(gen, m, k).to(dev)
+    w = (1 + 0.1 * torch.randn(k, generator=gen)).to(torch.bfloat16).to(dev)
+    s, y = pkg.ops.add_rmsnorm(x, r, w, 1e-5)
+    got = torch.empty_like(y)
+    target = x if into == "x" else r
+    status = pkg.library().lse_add_rmsnorm(
+        x.data_ptr(), k, r.data_ptr(), k, w.data_ptr(), 1e-5, target.data_ptr(), got.data_ptr(), m,
+        k, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert status == 0 and torch.equal(target, s) and torch.equal(got, y)
+
+
 def test_rejections(pkg, dev):
     x = torch.zeros(2, 16392, dtype=torch.bfloat16, device=dev)
     with pytest.raises(RuntimeError, match="range"):

@@ -517,6 +517,8 @@ def add_rmsnorm(
                  "the residual must be bf16 and of x's shape")
         r2, s = _rows(residual, k), torch.empty(x.shape, dtype=torch.bfloat16, device=dev)
     w = weight.contiguous()
+    if w.data_ptr() % 16:  # a piece of a flat parameter buffer
+        w = w.clone()
     _lib.check(
         _lib.library().lse_add_rmsnorm(
             x2.data_ptr(), x2.stride(0) if m > 1 else k,

@@ -91,6 +91,14 @@ def test_add_rmsnorm_in_place(pkg, dev, m, k, into):
     assert status == 0 and torch.equal(target, s) and torch.equal(got, y)
 
 
+def test_add_rmsnorm_takes_a_piece_of_a_flat_weight(pkg, dev):
+    """A contiguous weight at an address no 16-byte load takes: the same result as its aligned copy."""
+    gen = torch.Generator().manual_seed(5)
+    x, flat = _bf16(gen, 3, 64).to(dev), _bf16(gen, 65).to(dev)
+    want = pkg.ops.add_rmsnorm(x, None, flat[1:].clone(), 1e-5)[1]
+    assert torch.equal(pkg.ops.add_rmsnorm(x, None, flat[1:], 1e-5)[1], want)
+
+
 def test_rejections(pkg, dev):
     x = torch.zeros(2, 16392, dtype=torch.bfloat16, device=dev)
     with pytest.raises(RuntimeError, match="range"):

@@ -45,6 +45,7 @@ import math
 
 import torch
 from torch import nn
+from torch.nn.modules import module as nn_module
 
 from . import _lib, ops
 from .int8_linear import Int8GateUp, Int8Linear, PackedBf16Linear
@@ -262,23 +263,23 @@ class DecodeRunner:
 
     def _add_norm(self, norm: nn.Module, x: torch.Tensor, residual: torch.Tensor | None):
         """(x + residual, norm(x + residual)), as one kernel where it can be."""
-        if self._fused:
+        if self._fused and x.dtype == torch.bfloat16 and (residual is None
+                                                          or residual.dtype == torch.bfloat16):
             return ops.add_rmsnorm(x, residual, norm.weight, norm.variance_epsilon)
         hidden = x if residual is None else residual + x
         return hidden, norm(hidden)
 
     def _fusable(self) -> bool:
         """Whether the rotary embedding, the K/V writes and the norms of this model run as the fused
-        kernels: bf16 on the GPU, plain LlamaRMSNorms without hooks, a head and a row size they
-        take."""
+        kernels: bf16 on the GPU, plain norms (`plain_norm`), a head and a row size they take."""
         model = self.model.model
         norms = [model.norm, *(n for layer in self.layers
                                for n in (layer.input_layernorm, layer.post_attention_layernorm))]
-        return (self.k_cache[0].is_cuda and self.head_dim % 16 == 0 and self.head_dim <= 1024
-                and norms[0].weight.shape[0] % 8 == 0
-                and norms[0].weight.shape[0] <= _lib.NORM_MAX_K
-                and all(type(n).__name__ == "LlamaRMSNorm" and n.weight.dtype == torch.bfloat16
-                        and not (n._forward_hooks or n._forward_pre_hooks) for n in norms))
+        cache, size = self.k_cache[0], model.embed_tokens.weight.shape[-1]
+        return (cache.is_cuda and self.head_dim % 16 == 0 and self.head_dim <= 1024
+                and size % 8 == 0 and size <= _lib.NORM_MAX_K
+                and all(plain_norm(n) and n.weight.shape == (size,)
+                        and n.weight.device == cache.device for n in norms))
 
     @torch.no_grad()
     def forward(self, tokens: torch.Tensor, start: int, rows: slice | None = None) -> torch.Tensor:
@@ -366,6 +367,23 @@ class DecodeRunner:
                 n = mod.out_features
                 total += 2 * k * n + 2 * m * k + 2 * m * n
         return total
+
+
+def plain_norm(norm: nn.Module) -> bool:
+    """Whether calling `norm` runs transformers' own LlamaRMSNorm.forward on a bf16 weight and nothing
+    else: no subclass or namesake, no forward replaced on the class or the instance, no hook of its own or
+    of every module. Only such a call may be replaced by a kernel."""
+    from transformers.models.llama.modeling_llama import LlamaRMSNorm
+
+    if type(norm) is not LlamaRMSNorm or "forward" in vars(norm):
+        return False
+    forward = LlamaRMSNorm.forward
+    own = (forward.__module__, forward.__qualname__) == (LlamaRMSNorm.__module__,
+                                                         "LlamaRMSNorm.forward")
+    hooks = (norm._forward_hooks or norm._forward_pre_hooks or nn_module._global_forward_hooks
+             or nn_module._global_forward_pre_hooks)
+    return (own and not hooks and norm.weight.dtype == torch.bfloat16
+            and norm.variance_epsilon >= 0.0)
 
 
 class SiluMul(nn.Module):

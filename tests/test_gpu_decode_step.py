@@ -152,3 +152,71 @@ def test_indexed_rows_write_their_cache(runner, dev, rows):
     assert torch.equal(got, want)
     for c, kv in caches:
         assert torch.equal(c[4:7, :, 36], kv)
+
+
+@torch.no_grad()
+def _unfused(r, tokens, start, rows):
+    """`DecodeRunner.forward` spelled out with the reference's eager operations: each block's residual
+    added before the next norm (decoder_hidden, model_runner.py:213-224)."""
+    nseq, ntok = tokens.shape
+    model = r.model.model
+    r._rows, r._fused = rows, False
+    if r.attention == "paged":
+        r._plan = r._paged_plan(start, start + ntok, nseq, ntok)
+    pos = torch.arange(start, start + ntok, device=tokens.device).repeat(nseq, 1)
+    hidden = model.embed_tokens(tokens.reshape(1, -1))
+    cos, sin = model.rotary_emb(hidden, pos.reshape(1, -1))
+    for i, layer in enumerate(r.layers):
+        normed = layer.input_layernorm(hidden)
+        hidden = hidden + r._attend(i, normed, (cos[0], sin[0]), start, nseq, ntok)
+        hidden = hidden + r._mlp(i, layer.post_attention_layernorm(hidden))
+    return model.norm(hidden)
+
+
+@pytest.mark.parametrize("attention", ["torch", "paged"])
+@pytest.mark.parametrize("ntok", [1, 3])
+def test_fused_kernels_against_the_eager_operations(runner, dev, attention, ntok):
+    """A forward with the fused kernels and one of eager operations, written in the reference's order,
+    from the same cache: the norms' sums of squares alone differ (in fp32), which moves few bf16
+    roundings; a norm, residual, position or row taken from the wrong place changes everything."""
+    runner.enable_paged()
+    runner.use_attention(attention)
+    try:
+        runner.use("bf16")
+        gen = torch.Generator().manual_seed(19)
+        tok = torch.randint(0, runner.model.config.vocab_size, (5, ntok), generator=gen).to(dev)
+        rows, at = slice(3, 8), slice(33, 33 + ntok)
+        got = runner.forward(tok, 33, rows)
+        assert runner._fused
+        written = [c[rows, :, at].clone() for c in (*runner.k_cache, *runner.v_cache)]
+        pools = [p.clone() for p in (*runner.k_pool, *runner.v_pool)]
+        want = _unfused(runner, tok, 33, rows)
+        rel = lambda a, b: float((a.float() - b.float()).norm() / b.float().norm())  # noqa: E731
+        assert rel(got, want) < 0.01
+        caches = [c[rows, :, at] for c in (*runner.k_cache, *runner.v_cache)]
+        for layer, (a, b) in enumerate(zip(written, caches)):
+            assert rel(a, b) < 0.01, f"cache {layer}"
+        for layer, (a, b) in enumerate(zip(pools, (*runner.k_pool, *runner.v_pool))):
+            assert rel(a, b) < 0.01, f"pool {layer}"
+        assert rel(runner.lm_head()(got[0]), runner.lm_head()(want[0])) < 0.01
+    finally:
+        runner.use_attention("torch")
+
+
+def test_a_norm_with_other_behaviour_is_called(runner, dev):
+    """A norm whose forward was replaced runs, and so does a hook on every module."""
+    runner.use("bf16")
+    tok = torch.full((2, 1), 7, device=dev)
+    norm, calls = runner.model.model.norm, []
+    norm.forward = lambda x: torch.zeros_like(x)
+    try:
+        assert not runner.forward(tok, 34, slice(0, 2)).any()
+    finally:
+        del norm.forward
+    handle = torch.nn.modules.module.register_module_forward_hook(
+        lambda mod, args, out: calls.append(mod))
+    try:
+        runner.forward(tok, 34, slice(0, 2))
+    finally:
+        handle.remove()
+    assert sum(mod is norm for mod in calls) == 1

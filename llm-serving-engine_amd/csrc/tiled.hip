@@ -895,6 +895,13 @@ constexpr double kTileEff16[kTileCands] = {1.0,  0.86, 0.87, 0.835, 0.6,
 // 128 x 128) measured 11-19 % faster.
 constexpr double kTileEff8[kTileCands] = {1.0,   0.76, 0.80, 0.72, 0.6,
                                           0.926, 0.75, 0.92, 0.87, 0.80};
+// W8A8 over few K steps: a block of the 192-row tile is alone on its CU, and its prologue and epilogue, which
+// two 128 x 128 blocks hide for each other, weigh more the shorter K is. Where the two meet (five rounds
+// of 128 x 128 against two) it measured, gate/up of I 8192 at 1025..1280 tokens, 128 x 128 / 192 x 256:
+// K 1024 33.7 / 37.9 us, 2048 49 / 52, 3072 74 / 78, 4096 94 / 95, 6144 138 / 132; plain N 5846, K 2304, 3136
+// tokens 77 / 82; N 5120, K 3072, 3552 tokens 70 / 68. W8A16 gained at every K.
+constexpr double kTileEff8Short192 = 0.85;
+constexpr int64_t kShortK = 3072, kShortKGlu = 4096;
 
 // One round of candidate i on every CU, in the cost model's units.
 template <bool I8>
@@ -903,7 +910,7 @@ static double tile_round_cost(int i) {
 }
 
 template <bool I8>
-static TiledShape tiled_shape(int64_t M, int64_t N, int cus, double* cost_out = nullptr,
+static TiledShape tiled_shape(int64_t M, int64_t N, int64_t K, int cus, double* cost_out = nullptr,
                               bool glu = false) {
   TiledShape best = kTileCand[0];
   double best_cost = 1e300;
@@ -914,7 +921,9 @@ static TiledShape tiled_shape(int64_t M, int64_t N, int cus, double* cost_out = 
     if (kTileCand[i].bm == 96 && (I8 || M > 96)) continue;  // W8A16, one block row only
     if (kTileCand[i].bm == 112 && (I8 || !glu)) continue;  // W8A16 gate/up only
     const int64_t blocks = ceil_div(M, kTileCand[i].bm) * ceil_div(N, kTileCand[i].bn);
-    const double cost = (double)ceil_div(blocks, (int64_t)cus) * tile_round_cost<I8>(i);
+    double cost = (double)ceil_div(blocks, (int64_t)cus) * tile_round_cost<I8>(i);
+    if (I8 && kTileCand[i].bm == 192 && K < (glu ? kShortKGlu : kShortK))
+      cost *= kTileEff8[i] / kTileEff8Short192;
     if (cost < best_cost * 0.999) {
       best_cost = cost;
       best = kTileCand[i];
@@ -1029,11 +1038,11 @@ static int tiled_splits(bool i8, int64_t M, int64_t N, int64_t K, int cus) {
 // tokens (8 splits) from 64 x 128 tiles at two splits, 50-55 us, to one 256 x 128 block row,
 // 39-47 us (W8A16).
 template <bool I8>
-static TiledShape split_tile(int64_t M, int64_t N, int splits, int cus) {
+static TiledShape split_tile(int64_t M, int64_t N, int64_t K, int splits, int cus) {
   const int64_t nb = ceil_div(N, 128);
   for (int bm : {64, 128, 256})
     if (ceil_div(M, (int64_t)bm) * nb * splits <= cus) return TiledShape{bm, 128};
-  return tiled_shape<I8>(M, N, cus);
+  return tiled_shape<I8>(M, N, K, cus);
 }
 
 int64_t tiled_workspace_bytes(bool i8, int64_t M, int64_t N, int64_t K) {
@@ -1066,7 +1075,7 @@ static int launch_tiled(const void* x, int64_t ldx, const int8_t* qp, const floa
   if (splits > 1) {
     if (!ws || ws_bytes < (int64_t)splits * M * kTileRows * ceil_div(N, kTileRows) * 4)
       return LSE_E_WORKSPACE;
-    const TiledShape sh = split_tile<I8>(M, N, splits, cus);
+    const TiledShape sh = split_tile<I8>(M, N, K, splits, cus);
     const int64_t mblocks = ceil_div(M, sh.bm);
     const int64_t blocks = mblocks * ceil_div(N, sh.bn);
     TiledArgs a{};
@@ -1098,7 +1107,7 @@ static int launch_tiled(const void* x, int64_t ldx, const int8_t* qp, const floa
     return launch_skinny_reduce_parts(I8, ws, s, sx, y, ldy, acc, M, N, splits, stream);
   }
   double cost = 0.0;
-  const TiledShape sh = tiled_shape<I8>(M, N, cus, &cost, glu > 0);
+  const TiledShape sh = tiled_shape<I8>(M, N, K, cus, &cost, glu > 0);
   // Bulk and tail: a 256-row or 256-column tile whose blocks leave a partial last round after
   // at least one full one runs its full rounds over the first columns, and the cost model's tile
   // for the rest of N runs as a second launch; taken when some such pair is modelled at least
@@ -1118,7 +1127,7 @@ static int launch_tiled(const void* x, int64_t ldx, const int8_t* qp, const floa
     const int64_t n_bulk = full * cus / mb * c.bn;
     if (n_bulk >= N) continue;
     double tail_cost = 0.0;
-    const TiledShape t = tiled_shape<I8>(M, N - n_bulk, cus, &tail_cost, glu > 0);
+    const TiledShape t = tiled_shape<I8>(M, N - n_bulk, K, cus, &tail_cost, glu > 0);
     const double total = full * tile_round_cost<I8>(i) + tail_cost;
     if (total < best) {
       best = total;

@@ -10,7 +10,9 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
+from helpers import bf16_bits, to_bf16_tensor
 from oracle import numerics as ora
 from test_gpu_attention import _case, _check, _run
 
@@ -155,3 +157,138 @@ def test_entries_in_order_of_length(pkg, dev, entries):
     o = _run(pkg, dev, pad)
     keep = pad["ql"] > 0
     np.testing.assert_array_equal(o[:, keep], base[:, keep])
+
+
+def _indexes(c, dev):
+    return [torch.from_numpy(np.ascontiguousarray(c[k], np.int32)).to(dev)
+            for k in ("table", "ctx", "qo", "qs", "ql")]
+
+
+@pytest.mark.parametrize("block_size", [16, 24])
+@pytest.mark.parametrize("pools", ["padded rows", "head-major blocks"])
+def test_layouts(pkg, dev, block_size, pools):
+    """q as columns of a stacked projection, token-major, with o in its order, and pools of other
+    strides: the bits of the contiguous call, long and short entries."""
+    entries = [(70, 30, 100), (1, 60, 61), (5, 0, 5), (64, 0, 64)]
+    c = _case_of([0, 3], 800 + block_size, entries, **WIDE, block_size=block_size)
+    want = _check(pkg, dev, c, "contiguous")
+    h, tokens, d = c["q"].shape
+    stacked = torch.zeros(tokens, (h + 20) * d, dtype=torch.bfloat16, device=dev)
+    q = stacked[:, :h * d].view(tokens, h, d).transpose(0, 1)
+    q.copy_(to_bf16_tensor(c["q"], dev))
+    kv = []
+    for name in ("kp", "vp"):
+        pool = to_bf16_tensor(c[name], dev)
+        blocks, slots, heads, _ = pool.shape
+        if pools == "padded rows":
+            view = torch.full((blocks, slots, heads, 2 * d), float("nan"), dtype=pool.dtype,
+                              device=dev)[..., :d]
+        else:
+            view = torch.empty(blocks, heads, slots, d, dtype=pool.dtype, device=dev).transpose(1, 2)
+        kv.append(view.copy_(pool))
+    o = pkg.ops.paged_attention_forward(q, *kv, *_indexes(c, dev), c["bs"], c["max_q_len"])
+    np.testing.assert_array_equal(bf16_bits(o), want)
+
+
+def _with_scale(pkg, dev, c, scale):
+    q, k, v = (to_bf16_tensor(c[n], dev) for n in ("q", "kp", "vp"))
+    table, ctx, qo, qs, ql = _indexes(c, dev)
+    o = torch.empty_like(q)
+    lib, (h, _, d), h_kv = pkg.library(), q.shape, k.shape[2]
+    shape = (len(ctx), h, h_kv, d)
+    nbytes = lib.lse_paged_attention_workspace_bytes(*shape, c["max_q_len"], table.shape[1], c["bs"])
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
+    status = lib.lse_paged_attention(
+        q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), v.data_ptr(), *k.stride()[:3],
+        table.data_ptr(), table.stride(0), ctx.data_ptr(), qo.data_ptr(), qs.data_ptr(),
+        ql.data_ptr(), o.data_ptr(), o.stride(0), o.stride(1), *shape, c["bs"], table.shape[1],
+        c["max_q_len"], scale, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert status == 0
+    return bf16_bits(o)
+
+
+def test_negative_and_zero_scales(pkg, dev):
+    """The C entry's softmax scale of either sign, and none: the bits of the negated and of zero queries
+    under a positive one, long and short entries."""
+    c = _case_of([0], 820, [(70, 30, 100), (5, 40, 45), (1, 99, 100)], **WIDE)
+    np.testing.assert_array_equal(_with_scale(pkg, dev, c, -0.125),
+                                  _with_scale(pkg, dev, dict(c, q=c["q"] ^ 0x8000), 0.125))
+    np.testing.assert_array_equal(_with_scale(pkg, dev, c, 0.0),
+                                  _with_scale(pkg, dev, dict(c, q=np.zeros_like(c["q"])), 0.125))
+
+
+@pytest.mark.parametrize("key", [0, 20, 64, 130])
+def test_infinite_scores(pkg, dev, key):
+    """A score of -inf leaves its key out; one of +inf makes the rows that see it NaN, and no other."""
+    c = _case_of([0, 1], 830, [(150, 0, 150), (64, 0, 64)], **WIDE)
+    c["q"][:, :, 0] = 0x3F80  # 1.0
+    clean = _run(pkg, dev, c)
+    at = (c["table"][0][key // c["bs"]], key % c["bs"])
+    c["kp"] = c["kp"].copy()
+    c["kp"][at[0], at[1], :, 0] = 0xFF80  # -inf
+    left_out = _run(pkg, dev, c)
+    golden, covered = ora.paged_attention_golden(
+        c["q"], np.where(c["kp"] == 0xFF80, np.uint16(0xFF7F), c["kp"]), c["vp"], c["table"],
+        c["ctx"], c["qo"], c["qs"], c["ql"], c["bs"])
+    if key == 0:  # its own row sees no other key
+        assert not (left_out[:, 0] & 0x7FFF).any()
+        covered = covered.copy()
+        covered[0] = False
+    vmax = float(np.abs(ora.bf16_bits_to_f32(c["vp"])).max())
+    ok, msg = ora.attention_within_tolerance(left_out, golden, vmax, covered)
+    assert ok, msg
+    c["kp"][at[0], at[1], :, 0] = 0x7F80  # +inf
+    o = ora.bf16_bits_to_f32(_run(pkg, dev, c))
+    assert np.isnan(o[:, key:150]).all()
+    np.testing.assert_array_equal(ora.f32_to_bf16_bits(o[:, :key]), clean[:, :key])
+    np.testing.assert_array_equal(ora.f32_to_bf16_bits(o[:, 150:]), clean[:, 150:])
+
+
+@pytest.mark.parametrize("bad", [0x7FC0, 0x7F80])
+def test_how_far_a_non_finite_v_row_reaches(pkg, dev, bad):
+    """NaN or infinity in a token's V: NaN or infinite for the rows that see it, no trace in the rows of
+    earlier row tiles (8 tokens of 16 heads), other K/V heads and other entries."""
+    c = _case_of([0, 1], 840, [(70, 0, 70), (64, 0, 64)], **WIDE)
+    clean = _run(pkg, dev, c)
+    token, head = 44, 3
+    vp = c["vp"].copy()
+    vp[c["table"][0][token // c["bs"]], token % c["bs"], head] = bad
+    o = _run(pkg, dev, c, vp=vp)
+    group = slice(16 * head, 16 * head + 16)
+    assert not np.isfinite(ora.bf16_bits_to_f32(o[group, token:70])).any()
+    same = np.ones(o.shape[:2], bool)
+    same[group, token // 8 * 8:70] = False
+    np.testing.assert_array_equal(o[same], clean[same])
+
+
+@pytest.mark.parametrize("max_q_len", [9000, 40000, 100000])
+def test_work_list_of_grouped_row_tiles(pkg, dev, max_q_len):
+    """A max_q_len whose row tiles exceed the work list's levels (1024) puts several tiles into one: the
+    same bits as with the exact one."""
+    c = _case_of([0, 2, 3], 850, [(150, 77, 227), (1, 300, 301), (64, 0, 64), (333, 0, 333)], **WIDE)
+    base = _check(pkg, dev, c, "exact max_q_len")
+    np.testing.assert_array_equal(_run(pkg, dev, dict(c, max_q_len=max_q_len)), base)
+
+
+def test_more_items_than_a_workgroup_lists_at_once(pkg, dev):
+    """1024 entries of 136 items: over 512 for each of 256 workgroups, so that the lists are filled twice.
+    Every entry has the bits it has in a call of 64."""
+    h, h_kv, d, n, count, bs = 32, 8, 128, 520, 1024, 16
+    gen = torch.Generator(device=dev).manual_seed(860)
+    bf16 = lambda *shape: torch.randn(*shape, generator=gen, device=dev,  # noqa: E731
+                                      dtype=torch.bfloat16)
+    blocks = -(-n // bs)
+    k, v, q = bf16(blocks, bs, h_kv, d), bf16(blocks, bs, h_kv, d), bf16(count * n, h, d)
+    full = lambda m, value: torch.full((m,), value, dtype=torch.int32, device=dev)  # noqa: E731
+
+    def run(rows, m):
+        table = torch.arange(blocks, dtype=torch.int32, device=dev).repeat(m, 1)
+        start = torch.arange(0, m * n, n, dtype=torch.int32, device=dev)
+        return pkg.ops.paged_attention_forward(rows.transpose(0, 1), k, v, table, full(m, n),
+                                               full(m, 0), start, full(m, n), bs, n).transpose(0, 1)
+
+    o = run(q, count)
+    for e in range(0, count, 64):
+        rows = slice(e * n, (e + 64) * n)
+        assert torch.equal(o[rows], run(q[rows], 64)), f"entries from {e}"

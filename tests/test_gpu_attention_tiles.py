@@ -87,6 +87,17 @@ def test_peaked_and_flat_scores(pkg, dev, log2_q):
     _check(pkg, dev, c, f"q x 2^{log2_q}")
 
 
+def _errors(pkg, dev, c):
+    """(relative error against fp64, the part of it that rounding the fp64 result to bf16 makes)."""
+    o = ora.bf16_bits_to_f32(_run(pkg, dev, c)).astype(np.float64)
+    golden, _ = ora.paged_attention_golden(c["q"], c["kp"], c["vp"], c["table"], c["ctx"], c["qo"],
+                                           c["qs"], c["ql"], c["bs"])
+    golden = np.asarray(golden, np.float64)
+    rounded = ora.bf16_bits_to_f32(ora.f32_to_bf16_bits(golden.astype(np.float32)))
+    rms = lambda a: float(np.sqrt((a ** 2).mean() / (golden ** 2).mean()))  # noqa: E731
+    return rms(o - golden), rms(rounded - golden)
+
+
 def test_the_largest_probabilities_are_exact(pkg, dev):
     """Few keys matter: each tile's largest probability is rounded to bf16 without error, so the
     relative error stays near that of the output's own rounding (0.00165). Over 1300 keys the other
@@ -94,13 +105,18 @@ def test_the_largest_probabilities_are_exact(pkg, dev):
     would all add 0.0014. The bound allows them 0.0007."""
     c = _case_of([0], 460, [(100, 1200, 1300)], **WIDE)
     c["q"] = ora.f32_to_bf16_bits(ora.bf16_bits_to_f32(c["q"]) * np.float32(3))
-    o = ora.bf16_bits_to_f32(_run(pkg, dev, c)).astype(np.float64)
-    golden, _ = ora.paged_attention_golden(c["q"], c["kp"], c["vp"], c["table"], c["ctx"], c["qo"],
-                                           c["qs"], c["ql"], c["bs"])
-    golden = np.asarray(golden, np.float64)
-    rounded = ora.bf16_bits_to_f32(ora.f32_to_bf16_bits(golden.astype(np.float32)))
-    rms = lambda a: float(np.sqrt((a ** 2).mean() / (golden ** 2).mean()))  # noqa: E731
-    assert rms(o - golden) <= np.hypot(rms(rounded - golden), 0.0007)
+    error, rounding = _errors(pkg, dev, c)
+    assert error <= np.hypot(rounding, 0.0007)
+
+
+@pytest.mark.parametrize("tokens", [80, 417])
+def test_rows_of_few_keys_keep_their_probabilities(pkg, dev, tokens):
+    """A fresh prompt, whose first rows are the largest: beside the output's rounding (0.0016) its
+    probabilities add 0.0003 at 80 tokens and 0.00075 at 417. Rounded to bf16 in those rows too they
+    would add 0.0010 and 0.0011; the bounds lie between."""
+    c = _case_of([0], 470 + tokens, [(tokens, 0, tokens)], h=128, h_kv=8)
+    error, rounding = _errors(pkg, dev, c)
+    assert error <= np.hypot(rounding, 0.0005 if tokens == 80 else 0.0009)
 
 
 def test_rows_that_see_no_key(pkg, dev):

@@ -287,9 +287,13 @@ int64_t lse_paged_attention_workspace_bytes(int64_t entries, int64_t H, int64_t 
  *   pass its bucket size). workspace as sized by lse_paged_attention_workspace_bytes.
  * Determinism: each row's keys are summed in a fixed order (1024-position chunks for entries of few
  *   query rows, two interleaved streams of 64-key tiles for long ones; which one an entry gets is
- *   decided by its own q_len and context_len), so a row's output does not depend on the other
- *   entries, the entry count, max_q_len or the table width (a graph bucket with q_len = 0 padding
- *   rows and a pool-wide table gives the bits an exact-width eager call gives).
+ *   decided by its own q_len and context_len and by the head counts), so a row's output does not
+ *   depend on the other entries, the entry count, max_q_len or the table width (a graph bucket with
+ *   q_len = 0 padding rows and a pool-wide table gives the bits an exact-width eager call gives). It may
+ *   depend, within the probabilities' rounding, on the q_len of the chunk that its prompt is cut into.
+ * Non-finite values: a key of score -inf is left out, one of +inf or NaN makes the rows that see it NaN;
+ *   infinity or NaN in a V row makes the rows that see it non-finite and may reach rows of the same
+ *   entry and K/V head up to 127 query rows (tokens x H / H_KV) before it, and no others.
  * Replaces: `paged_attention_forward` (src/llm_serving_engine/kernels/flash_attention.py:
  *   287-332, the Triton kernel `paged_attention_2` at :201-284), called from
  *   `ModelRunner.attend_paged` (model_runner.py:357-363).

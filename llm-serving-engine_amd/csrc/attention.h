@@ -27,7 +27,7 @@ struct PagedAttnArgs {
   int entries, H, HKV, G, block_size, max_q_len;
   int bs_shift;      // log2(block_size) when it is a power of two, else -1
   int tq;            // query tokens per tile: floor(16 / G)
-  int qtiles;        // ceil(max_q_len / tq)
+  int qtiles;        // query tiles of the longest entry of this kernel
   int parts;         // 1: a workgroup folds every chunk of its item; > 1: one chunk per workgroup
   int sorted;        // entries are taken in descending order of context length...
   int first_round;   // ...and, where > 0, those from this rank on in ascending order

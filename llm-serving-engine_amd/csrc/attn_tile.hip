@@ -34,10 +34,9 @@
 // Order of summation: tiles 2 j + s of stream s in order, then the two streams. It depends on the
 // row's own entry only.
 //
-// Measured on MI355X: three fresh prompts of 1285-1321 tokens, 32 heads over 8, 268 -> 71 us (590
-// TFLOP/s of the causal half; a dense bf16 product of 8192^3 reaches 1434); a 735-token chunk behind
-// 1291 positions beside 40 decode rows, 24 heads over 8, 170 -> 91 us, of which this kernel 38 (and
-// attention.hip's, with its entries in order of length, 53). A phase takes 1300-1600 clocks of which
+// Measured on MI355X, against the key-streaming kernel: three fresh prompts of 1285-1321 tokens, 32
+// heads over 8, 268 -> 74 us (570 TFLOP/s of the causal half; a dense bf16 product of 8192^3 reaches
+// 1434); a 735-token chunk behind 1291 positions, 24 heads over 8, 107 -> 38. A phase takes 1300-1600 clocks of which
 // 1024 are MFMA issue; an item's first loads and its merge another 10000 or so, about a third of
 // the time at these prompt lengths. Without gain, against 66-68 us: the next item's first loads
 // issued before the merge (69 us); the tiles of consecutive items in one pipeline (73-105 us: the

@@ -875,7 +875,8 @@ static const void* tiled_kernel_for(const TiledShape& sh, bool decode = false,
 // 37.6-38.8 us. Measured only there, so only launches of one such block row consider it.
 // The 224-, 192- and 112-row tiles (256 x 256 and 128 x 256 schedules over fewer token rows, ROWS) are
 // for token counts just past a multiple of a block row, where most of the last one would be
-// padding: their MFMAs shrink with the rows, their loads, barriers and dequantization do not, hence
+// padding: their MFMAs shrink with the rows, their load instructions, barriers and dequantization do
+// not (loads of rows past the tile's are out of the resource's range and request no memory), hence
 // the lower efficiencies, fitted so that none is picked where it measured slower. On MI355X, fused
 // gate/up (K 3072, N 16384) at 600 / 700 tokens 72.9 -> 63.2 / 75.6 -> 62 us in W8A16 and 39.7 ->
 // 35.8 / 40.4 -> 37.2 in W8A8; (K 4096, N 28672) at 300 / 1700 tokens 98 -> 86 / 406 -> 340 us; q/k/v
